@@ -1256,6 +1256,7 @@ namespace {
 
 struct BatchGroup {
     int dim = 0, n = 0, precision = 0;
+    bool generic = false;                // FP64 with the Kennedy-Gruber or Ismail-Roe flux
     int tile = -1;                       // batched tile (batch_tile); -1: per-instance launches
     std::vector<int> inst;               // instance indices
     BatchBlock *blocks = nullptr;        // device block table
@@ -1310,6 +1311,8 @@ static void batch_free_groups(dgx_batch *b)
     b->events.clear();
 }
 
+static bool batch_generic(const dgx_ctx *c) { return c->P.precision == DGX_FP64 && c->pc.two_point < 2; }
+
 static bool batch_line_eligible(const dgx_ctx *c)
 {
     return c->P.use_split_form && c->P.pde == DGX_EULER && !c->has_boundary && !c->curv;
@@ -1334,7 +1337,7 @@ static int group_table(dgx_batch *b, const BatchGroup &g, int epb, BatchBlock **
 static int batch_blocks(dgx_batch *b, BatchGroup &g, int tile)
 {
     int epb = 0;
-    int rc = launch_line_batch(g.dim, g.n, g.precision, tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &epb);
+    int rc = launch_line_batch(g.dim, g.n, g.precision, g.generic, tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &epb);
     if (rc) return rc;
     (void)hipFree(g.blocks);
     g.blocks = nullptr;
@@ -1349,7 +1352,7 @@ static int batch_blocks(dgx_batch *b, BatchGroup &g, int tile)
 static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
 {
     if (b->forced_tile >= 0 && batch_blocks(b, g, b->forced_tile) == DGX_OK) return DGX_OK;
-    const long key = ((long)g.dim * 16 + g.n) * 4 + g.precision;
+    const long key = (((long)g.dim * 16 + g.n) * 4 + g.precision) * 2 + g.generic;
     for (auto &kv : g_variant_cache)
         if (kv.first == key) return batch_blocks(b, g, kv.second);
     // the group's own first-stage launch: it reads u_n and writes only the accumulator and the
@@ -1364,7 +1367,7 @@ static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
     std::vector<std::pair<int, std::pair<BatchBlock *, int>>> tables;  // epb -> (table, blocks)
     for (int tile = 0; tile < batch_tile_count(g.dim); ++tile) {
         int epb = 0;
-        if (launch_line_batch(g.dim, g.n, g.precision, tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &epb))
+        if (launch_line_batch(g.dim, g.n, g.precision, g.generic, tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &epb))
             continue;  // tile does not fit this shape
         int t = -1;
         for (size_t k = 0; k < tables.size(); ++k)
@@ -1386,7 +1389,7 @@ static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
         for (size_t k = 0; k < cand.size(); ++k) {
             const auto &tb = tables[table[k]].second;
             BHIPCHK(hipEventRecord(e0, b->stream));
-            if (launch_line_batch(g.dim, g.n, g.precision, cand[k], tb.first, tb.second, pa, g.pcs, ops, b->stream,
+            if (launch_line_batch(g.dim, g.n, g.precision, g.generic, cand[k], tb.first, tb.second, pa, g.pcs, ops, b->stream,
                                   nullptr))
                 return DGX_ERR_HIP;
             BHIPCHK(hipEventRecord(e1, b->stream));
@@ -1490,7 +1493,7 @@ int dgx_batch_tile(const dgx_batch *b, int i, int *elements_per_block, int *wave
     const bool fast = c->P.precision == DGX_MIXED;
     const BatchTile t = batch_tile(c->dim, fast, v - 1);
     *waves_bound = t.waves;
-    return launch_line_batch(c->dim, c->n, c->P.precision, v - 1, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
+    return launch_line_batch(c->dim, c->n, c->P.precision, batch_generic(c), v - 1, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
                              elements_per_block, threads_per_block);
 }
 
@@ -1525,13 +1528,14 @@ int dgx_batch_allocate(dgx_batch *b, int method, const double *dt)
         if (!batch_line_eligible(c)) continue;
         BatchGroup *g = nullptr;
         for (BatchGroup &h : b->groups)
-            if (h.dim == c->dim && h.n == c->n && h.precision == c->P.precision) g = &h;
+            if (h.dim == c->dim && h.n == c->n && h.precision == c->P.precision && h.generic == batch_generic(c)) g = &h;
         if (!g) {
             b->groups.emplace_back();
             g = &b->groups.back();
             g->dim = c->dim;
             g->n = c->n;
             g->precision = c->P.precision;
+            g->generic = batch_generic(c);
         }
         g->inst.push_back(i);
     }
@@ -1585,7 +1589,7 @@ int dgx_batch_allocate(dgx_batch *b, int method, const double *dt)
             if (k && hipStreamWaitEvent(gs, ev[0], 0) != hipSuccess) rc = DGX_ERR_HIP;
             const Ops1D &ops = b->inst[g.inst[0]]->ops;
             if (!rc)
-                rc = launch_line_batch(g.dim, g.n, g.precision, g.tile, g.blocks, g.nblocks, g.args[st], g.pcs, ops,
+                rc = launch_line_batch(g.dim, g.n, g.precision, g.generic, g.tile, g.blocks, g.nblocks, g.args[st], g.pcs, ops,
                                        gs, nullptr);
             if (!rc && k && hipEventRecord(ev[k], gs) != hipSuccess) rc = DGX_ERR_HIP;
         }
@@ -1775,6 +1779,7 @@ static int server_advance(dgx_server *s)
     }
     struct G {
         int dim, n, precision, tile, epb;
+        bool generic;
         std::vector<int> members;
         int64_t off_blocks, off_pcs, off_args;
         int nblocks;
@@ -1786,20 +1791,21 @@ static int server_advance(dgx_server *s)
         if (!batch_line_eligible(c)) continue;
         G *g = nullptr;
         for (G &x : groups)
-            if (x.dim == c->dim && x.n == c->n && x.precision == c->P.precision) g = &x;
+            if (x.dim == c->dim && x.n == c->n && x.precision == c->P.precision && x.generic == batch_generic(c)) g = &x;
         if (!g) {
             G x{};
             x.dim = c->dim;
             x.n = c->n;
             x.precision = c->P.precision;
-            const long key = ((long)x.dim * 16 + x.n) * 4 + x.precision;
+            x.generic = batch_generic(c);
+            const long key = (((long)x.dim * 16 + x.n) * 4 + x.precision) * 2 + x.generic;
             x.tile = 0;
             for (auto &kv : g_variant_cache)
                 if (kv.first == key) x.tile = kv.second;
-            if (launch_line_batch(x.dim, x.n, x.precision, x.tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
+            if (launch_line_batch(x.dim, x.n, x.precision, x.generic, x.tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
                                   &x.epb) != DGX_OK) {
                 x.tile = 0;
-                launch_line_batch(x.dim, x.n, x.precision, 0, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &x.epb);
+                launch_line_batch(x.dim, x.n, x.precision, x.generic, 0, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &x.epb);
             }
             groups.push_back(x);
             g = &groups.back();
@@ -1847,7 +1853,7 @@ static int server_advance(dgx_server *s)
         for (G &g : groups) {
             const int m = (int)g.members.size();
             const Ops1D &ops = s->active[g.members[0]].c->ops;
-            int rc = launch_line_batch(g.dim, g.n, g.precision, g.tile, (const BatchBlock *)(s->stage_dev + g.off_blocks),
+            int rc = launch_line_batch(g.dim, g.n, g.precision, g.generic, g.tile, (const BatchBlock *)(s->stage_dev + g.off_blocks),
                                        g.nblocks, (const StageArgs *)(s->stage_dev + g.off_args) + st * m,
                                        (const PhysConst *)(s->stage_dev + g.off_pcs), ops, s->stream, nullptr);
             if (rc) {

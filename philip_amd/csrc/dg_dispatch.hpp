@@ -24,14 +24,37 @@ inline int check_launch(dgx_ctx *c, const char *what)
     return DGX_OK;
 }
 
+// Split-form Euler on the box: with boundary faces or without, in FP64 with a kernel of its own for
+// the Kennedy-Gruber and Ismail-Roe fluxes.
+template <int D, int N, typename T>
+void line_dn(dgx_ctx *c, const StageArgs &a)
+{
+    using LG = LineGeoS<D, N, T>;
+    auto go = [&](auto bc, auto gc) {
+        constexpr bool BND = decltype(bc)::value, GEN = decltype(gc)::value;
+        const dim3 grid((c->ncells + LG::EPB - 1) / LG::EPB), block(LG::BLOCK);
+        if constexpr (line_waves<D, N, T>() > 0)
+            hipLaunchKernelGGL((line_kernel_wb<D, N, T, line_waves<D, N, T>(), BND, GEN>), grid, block, 0, c->stream,
+                               a, c->ops, c->pc);
+        else
+            hipLaunchKernelGGL((line_kernel<D, N, T, BND, GEN>), grid, block, 0, c->stream, a, c->ops, c->pc);
+    };
+    auto pick = [&](auto gc) {
+        if (c->has_boundary) go(std::true_type{}, gc);
+        else go(std::false_type{}, gc);
+    };
+    if constexpr (std::is_same<T, double>::value) {
+        if (c->pc.two_point < 2) return pick(std::true_type{});
+    }
+    pick(std::false_type{});
+}
+
 template <int D, int N, typename T>
 void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
 {
     const bool split = c->P.use_split_form != 0;
     const bool nsv = c->P.pde == DGX_NAVIER_STOKES;
     const bool bnd = c->has_boundary;
-    using LG = LineGeoS<D, N, T>;
-    const dim3 lgrid((c->ncells + LG::EPB - 1) / LG::EPB), lblock(LG::BLOCK);
     if (c->curv) {  // curvilinear grid: stage2_kernel with the metric terms, boundaries included
         if constexpr (D == 3) {
             if (nsv) {
@@ -62,8 +85,6 @@ void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
                 hipLaunchKernelGGL((stage2_kernel<D, N, false, true, T, true>), grid, block, 0, c->stream, a,
                                    c->ops, c->pc);
         } else if (split && nsv) {
-            // mixed: line kernel with the viscous terms; FP64: stage2_kernel (the FP64 line
-            // variant needs ~85 KB of LDS per block at p=5 and ran slower at one block per CU)
             if constexpr (std::is_same<T, float>::value) {
                 using LV = LineGeoK<D, N, T, true>;
                 const dim3 vgrid((c->ncells + LV::EPB - 1) / LV::EPB), vblock(LV::BLOCK);
@@ -79,19 +100,7 @@ void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
         else if (!split && nsv)
             hipLaunchKernelGGL((stage2_kernel<D, N, false, true, T>), grid, block, 0, c->stream, a, c->ops, c->pc);
         else if (split) {
-            if constexpr (line_waves<D, N, T>() > 0) {
-                if (bnd)
-                    hipLaunchKernelGGL((line_kernel_wb<D, N, T, line_waves<D, N, T>(), true>), lgrid, lblock, 0,
-                                       c->stream, a, c->ops, c->pc);
-                else
-                    hipLaunchKernelGGL((line_kernel_wb<D, N, T, line_waves<D, N, T>()>), lgrid, lblock, 0,
-                                       c->stream, a, c->ops, c->pc);
-            } else {
-                if (bnd)
-                    hipLaunchKernelGGL((line_kernel<D, N, T, true>), lgrid, lblock, 0, c->stream, a, c->ops, c->pc);
-                else
-                    hipLaunchKernelGGL((line_kernel<D, N, T>), lgrid, lblock, 0, c->stream, a, c->ops, c->pc);
-            }
+            line_dn<D, N, T>(c, a);
         } else if (bnd) {
             hipLaunchKernelGGL((stage2_kernel<D, N, false, false, T, true>), grid, block, 0, c->stream, a, c->ops,
                                c->pc);
@@ -100,10 +109,7 @@ void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
         }
     } else {
         if (split) {
-            if (bnd)
-                hipLaunchKernelGGL((line_kernel<D, N, T, true>), lgrid, lblock, 0, c->stream, a, c->ops, c->pc);
-            else
-                hipLaunchKernelGGL((line_kernel<D, N, T>), lgrid, lblock, 0, c->stream, a, c->ops, c->pc);
+            line_dn<D, N, T>(c, a);
         } else if (bnd) {
             hipLaunchKernelGGL((stage2_kernel<D, N, false, false, T, true>), grid, block, 0, c->stream, a, c->ops,
                                c->pc);
@@ -164,7 +170,7 @@ int launch_aux_dn(dgx_ctx *c, const double *u)
     return check_launch(c, "aux_kernel");
 }
 
-template <int D, int N, typename T, int ES, int W, bool XJ>
+template <int D, int N, typename T, int ES, int W, bool XJ, bool GEN>
 int line_batch_es(const BatchBlock *blocks, int nblocks, const StageArgs *args, const PhysConst *pcs,
                   const Ops1D &ops, hipStream_t st, int *epb, int *threads)
 {
@@ -176,23 +182,23 @@ int line_batch_es(const BatchBlock *blocks, int nblocks, const StageArgs *args, 
         if (threads) *threads = LG::BLOCK;
         if (!blocks) return DGX_OK;  // query only
         if constexpr (W > 0)
-            hipLaunchKernelGGL((line_kernel_batch_wb<D, N, T, ES, W, XJ>), dim3(nblocks), dim3(LG::BLOCK), 0, st,
+            hipLaunchKernelGGL((line_kernel_batch_wb<D, N, T, ES, W, XJ, GEN>), dim3(nblocks), dim3(LG::BLOCK), 0, st,
                                blocks, args, pcs, ops);
         else
-            hipLaunchKernelGGL((line_kernel_batch<D, N, T, ES, XJ>), dim3(nblocks), dim3(LG::BLOCK), 0, st, blocks,
+            hipLaunchKernelGGL((line_kernel_batch<D, N, T, ES, XJ, GEN>), dim3(nblocks), dim3(LG::BLOCK), 0, st, blocks,
                                args, pcs, ops);
         return hipGetLastError() == hipSuccess ? DGX_OK : DGX_ERR_HIP;
     }
 }
 
-template <int D, int N, typename T>
+template <int D, int N, typename T, bool GEN>
 int line_batch_t(int tile, const BatchBlock *blocks, int nblocks, const StageArgs *args, const PhysConst *pcs,
                  const Ops1D &ops, hipStream_t st, int *epb, int *threads)
 {
     constexpr bool F = std::is_same<T, float>::value;
 #define LBT_CASE(V)                                                                                              \
     case V:                                                                                                      \
-        return line_batch_es<D, N, T, batch_tile(D, F, V).es, batch_tile(D, F, V).waves, batch_tile(D, F, V).xj>( \
+        return line_batch_es<D, N, T, batch_tile(D, F, V).es, batch_tile(D, F, V).waves, batch_tile(D, F, V).xj, GEN>( \
             blocks, nblocks, args, pcs, ops, st, epb, threads);
     if constexpr (D == 2) {
         switch (tile) {
@@ -210,13 +216,14 @@ int line_batch_t(int tile, const BatchBlock *blocks, int nblocks, const StageArg
 }
 
 template <int D, int N>
-int line_batch_dn(int precision, int tile, const BatchBlock *blocks, int nblocks, const StageArgs *args,
+int line_batch_dn(int precision, bool generic, int tile, const BatchBlock *blocks, int nblocks, const StageArgs *args,
                   const PhysConst *pcs, const Ops1D &ops, hipStream_t st, int *epb, int *threads)
 {
     if (tile < 0 || tile >= batch_tile_count(D)) return DGX_ERR_UNSUPPORTED;
     if (precision == DGX_MIXED)
-        return line_batch_t<D, N, float>(tile, blocks, nblocks, args, pcs, ops, st, epb, threads);
-    return line_batch_t<D, N, double>(tile, blocks, nblocks, args, pcs, ops, st, epb, threads);
+        return line_batch_t<D, N, float, false>(tile, blocks, nblocks, args, pcs, ops, st, epb, threads);
+    if (generic) return line_batch_t<D, N, double, true>(tile, blocks, nblocks, args, pcs, ops, st, epb, threads);
+    return line_batch_t<D, N, double, false>(tile, blocks, nblocks, args, pcs, ops, st, epb, threads);
 }
 
 // explicit instantiation (in dg_inst_n<NN>.hip) and its extern declaration (in dg_launch.hip)
@@ -224,9 +231,9 @@ int line_batch_dn(int precision, int tile, const BatchBlock *blocks, int nblocks
     PREFIX template int launch_stage_dn<2, NN>(dgx_ctx *, const StageArgs &);                              \
     PREFIX template int launch_stage_dn<3, NN>(dgx_ctx *, const StageArgs &);                              \
     PREFIX template int launch_aux_dn<3, NN>(dgx_ctx *, const double *);                                   \
-    PREFIX template int line_batch_dn<2, NN>(int, int, const BatchBlock *, int, const StageArgs *,          \
+    PREFIX template int line_batch_dn<2, NN>(int, bool, int, const BatchBlock *, int, const StageArgs *,          \
                                              const PhysConst *, const Ops1D &, hipStream_t, int *, int *);   \
-    PREFIX template int line_batch_dn<3, NN>(int, int, const BatchBlock *, int, const StageArgs *,          \
+    PREFIX template int line_batch_dn<3, NN>(int, bool, int, const BatchBlock *, int, const StageArgs *,          \
                                              const PhysConst *, const Ops1D &, hipStream_t, int *, int *);
 
 } // namespace dgx

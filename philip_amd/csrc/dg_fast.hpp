@@ -6,8 +6,8 @@
 // speed, enthalpy) are computed once per node and reused by every pair and
 // face that touches the node.  In float the reciprocals, square roots and
 // logarithms are the hardware v_rcp_f32 / v_sqrt_f32 / v_log_f32 instructions;
-// in double the reciprocal is v_rcp_f64 with two Newton-Raphson steps, square
-// root and logarithm the library's double routines.
+// in double the reciprocal is v_rcp_f64 with a third-order step, the square root v_rsq_f64 with
+// Newton steps, the logarithm the library's double routine.
 //
 //   ec_flux_fast   Chandrashekar / Ranocha two-point flux (euler.cpp:709-807):
 //                  log means from f = (a-b)/(a+b), and 1/(2 beta_ln (gamma-1))
@@ -17,7 +17,17 @@
 //                  332-480) with Roe averages from sqrt(rho) of each side.
 //   num_flux_fast  baseline (central or two-point) + dissipation (LxF / Roe)
 //                  (convective_numerical_flux.cpp:34-54).
+//
+// The FP64 path's VALU issue is what its stage kernels spend most of their time on, so its
+// versions (the *64 functions) are arranged for fewer instructions than the float ones: one
+// reciprocal serves both 1/(rho1+rho2) and 1/(b1+b2), 1/F_rho comes from its expansion and one
+// Newton step, |avg v|^2 - avg |v|^2 / 2 is v1.v2 / 2, and a node's 1/rho and 1/p come from one
+// reciprocal.  Every sum over the two sides is written so that exchanging them and turning the
+// normal around gives the exact negative, so a face evaluated from either side needs no
+// selection of an owner.  They take a direction K or (CV) a normal / cofactor column nv.
 #pragma once
+#include <type_traits>
+
 #include "dg_physics.hpp"
 
 namespace dgx {
@@ -30,19 +40,38 @@ template <> struct Fast<float> {
     static __device__ __forceinline__ float log_(float x) { return __logf(x); }
 };
 template <> struct Fast<double> {
-    // v_rcp_f64 refined by two Newton-Raphson steps r <- r + r (1 - x r): v_rcp_f64 alone is within
-    // 4.6e-8 of 1/x, one step within 11 ulp, two steps gave the correctly rounded 1/x for all of 2^20
-    // samples over [e^-7, e^7] on gfx950 -- at half the instructions of the IEEE division sequence
-    // (FP64 stage kernel at p=3: 206 -> 197 us per stage; one step only would save 2 %)
+    // v_rcp_f64 (within 4.6e-8 of 1/x) refined by one third-order step r (1 + e + e^2), e = 1 - x r:
+    // the remaining relative error is e^3 ~ 1e-22, so the result is rounded once, at one FMA less
+    // than two Newton-Raphson steps
     static __device__ __forceinline__ double rcp(double x)
     {
-        double r = __builtin_amdgcn_rcp(x);
-        double e = __builtin_fma(-x, r, 1.0);
-        r = __builtin_fma(r, e, r);
-        e = __builtin_fma(-x, r, 1.0);
-        return __builtin_fma(r, e, r);
+        const double r = __builtin_amdgcn_rcp(x);
+        const double e = __builtin_fma(-x, r, 1.0);
+        const double t = __builtin_fma(e, e, e);
+        return __builtin_fma(r, t, r);
     }
-    static __device__ __forceinline__ double sqrt_(double x) { return sqrt(x); }
+    // sqrt(x) and 1/sqrt(x) from v_rsq_f64 by one coupled Newton (Goldschmidt) step and one residual
+    // correction each; no scaling (x is a density, a squared sound speed or a squared area).
+    // x = 0 and x = inf, whose products are NaN, are returned as they are.
+    static __device__ __forceinline__ void sqrt_rsqrt(double x, double *root, double *inv)
+    {
+        const double y = __builtin_amdgcn_rsq(x);
+        double g = x * y, h = 0.5 * y;
+        const double r = __builtin_fma(-h, g, 0.5);
+        g = __builtin_fma(g, r, g);
+        h = __builtin_fma(h, r, h);
+        const double d = __builtin_fma(-g, g, x);
+        g = __builtin_fma(d, h, g);
+        *root = __builtin_amdgcn_class(x, 0x260) ? x : g;  // -0, +0, +inf
+        const double q = __builtin_fma(-h, g, 0.5);
+        *inv = 2.0 * __builtin_fma(h, q, h);
+    }
+    static __device__ __forceinline__ double sqrt_(double x)
+    {
+        double g, h;
+        sqrt_rsqrt(x, &g, &h);
+        return g;
+    }
     static __device__ __forceinline__ double log_(double x) { return log(x); }
 };
 #else
@@ -53,7 +82,13 @@ template <typename T> struct FastHost {
     static inline T log_(T x) { return std::log(x); }
 };
 template <> struct Fast<float> : FastHost<float> {};
-template <> struct Fast<double> : FastHost<double> {};
+template <> struct Fast<double> : FastHost<double> {
+    static inline void sqrt_rsqrt(double x, double *root, double *inv)
+    {
+        *root = std::sqrt(x);
+        *inv = 1.0 / *root;
+    }
+};
 #endif
 template <typename T> __device__ __forceinline__ T frcp(T x) { return Fast<T>::rcp(x); }
 template <typename T> __device__ __forceinline__ T fsqrt(T x) { return Fast<T>::sqrt_(x); }
@@ -84,10 +119,27 @@ template <typename T> __device__ __forceinline__ FastConst<T> fast_const(const P
     return f;
 }
 
-// Fills every field of q from q.u; beta is rho/(2p) (Chandrashekar) or rho/p (Ranocha).
+// Fills every field of q from q.u; beta is rho/(2p) (Chandrashekar) or rho/p (Ranocha).  In double
+// 1/rho and 1/p = (g-1)^-1 rho / e, e = rho E - |m|^2/2, come from one reciprocal 1/(rho e), and
+// |v|^2, which the FP64 fluxes do not use, is left out.
 template <typename T, int D>
 __device__ __forceinline__ void node_fill(NodeC<T, D> &q, const FastConst<T> &fc)
 {
+    if constexpr (std::is_same<T, double>::value) {
+        double m2 = q.u[1] * q.u[1];
+        for (int k = 1; k < D; ++k) m2 += q.u[1 + k] * q.u[1 + k];
+        const double e = q.u[0] * q.u[D + 1] - 0.5 * m2;
+        const double r = frcp<double>(q.u[0] * e);
+        const double ir = r * e;
+        for (int k = 0; k < D; ++k) q.vel[k] = q.u[1 + k] * ir;
+        q.p = fc.gamm1 * (e * ir);
+        const double rp = fc.inv_gamm1 * (q.u[0] * q.u[0]) * (q.u[0] * r);
+        q.b = (fc.two_point == 3) ? rp : 0.5 * rp;
+        q.sr = fsqrt<double>(q.u[0]);
+        q.c = fsqrt<double>(fc.gam * q.p * ir);
+        q.h = (q.u[D + 1] + q.p) * ir;
+        return;
+    }
     const T ir = frcp<T>(q.u[0]);
     T v2 = T(0);
     for (int k = 0; k < D; ++k) {
@@ -146,12 +198,116 @@ __device__ __forceinline__ void ec_flux_fast(const T rho1, const T *v1, const T 
     if (ra) f[D + 1] -= T(0.5) * (p1 * v1[K] + p2 * v2[K]);
 }
 
+// The same in double (Chandrashekar / Ranocha), along e_K or (CV) contracted with nv.  1/F_rho: the
+// expansion of x / atanh x to u^3 is within 1e-9 of it for u < 1e-2, one Newton step squares that.
+template <int D, int K, bool CV>
+__device__ __forceinline__ void ec_flux64(const NodeC<double, D> &a, const NodeC<double, D> &b, const double *nv,
+                                          const FastConst<double> &fc, double *f)
+{
+    const bool ra = (fc.two_point == 3);
+    const double sr = a.u[0] + b.u[0], sb = a.b + b.b;
+    const double t = frcp<double>(sr * sb);
+    const double isr = t * sb, isb = t * sr;
+    const double fr = (a.u[0] - b.u[0]) * isr, fb = (a.b - b.b) * isb;
+    const double ur = fr * fr, ub = fb * fb;
+    double Fr = 1.0 + ur * (1.0 / 3.0 + ur * (1.0 / 5.0 + ur * (1.0 / 7.0)));
+    double Fb = 1.0 + ub * (1.0 / 3.0 + ub * (1.0 / 5.0 + ub * (1.0 / 7.0)));
+    const double g = 1.0 - ur * (1.0 / 3.0 + ur * (4.0 / 45.0 + ur * (44.0 / 945.0)));
+    double iFr = g + g * (1.0 - Fr * g);
+    if (__builtin_expect(!(ur < 1.0e-2 && ub < 1.0e-2), 0)) {
+        // larger over smaller: the same bits whichever side is a
+        if (!(ur < 1.0e-2)) {
+            const bool gt = a.u[0] > b.u[0];
+            const double hi = gt ? a.u[0] : b.u[0], lo = gt ? b.u[0] : a.u[0];
+            Fr = 0.5 * flog<double>(hi * frcp<double>(lo)) * frcp<double>(fab<double>(fr));
+            iFr = frcp<double>(Fr);
+        }
+        if (!(ub < 1.0e-2)) {
+            const bool gt = a.b > b.b;
+            const double hi = gt ? a.b : b.b, lo = gt ? b.b : a.b;
+            Fb = 0.5 * flog<double>(hi * frcp<double>(lo)) * frcp<double>(fab<double>(fb));
+        }
+    }
+    double w[D], dot = a.vel[0] * b.vel[0], wn = 0.0;
+    for (int k = 0; k < D; ++k) w[k] = a.vel[k] + b.vel[k];
+    for (int k = 1; k < D; ++k) dot += a.vel[k] * b.vel[k];
+    if constexpr (CV) {
+        wn = w[0] * nv[0];
+        for (int k = 1; k < D; ++k) wn += w[k] * nv[k];
+    } else {
+        wn = w[K];
+    }
+    double p_hat, H;
+    if (ra) {
+        p_hat = 0.5 * (a.p + b.p);
+        H = 2.0 * (Fb * isb * fc.inv_gamm1) + 4.0 * p_hat * (Fr * isr);
+    } else {
+        p_hat = 0.5 * sr * isb;
+        H = isb * (Fb * fc.inv_gamm1 + Fr);
+    }
+    H += 0.5 * dot;
+    const double m = 0.25 * sr * iFr * wn, hm = 0.5 * m;
+    f[0] = m;
+    if constexpr (CV) {
+        for (int vd = 0; vd < D; ++vd) f[1 + vd] = hm * w[vd] + p_hat * nv[vd];
+    } else {
+        for (int vd = 0; vd < D; ++vd) f[1 + vd] = (vd == K) ? hm * w[vd] + p_hat : hm * w[vd];
+    }
+    f[D + 1] = m * H;
+    if (ra) {
+        double pa, pb;
+        if constexpr (CV) {
+            double va = a.vel[0] * nv[0], vb = b.vel[0] * nv[0];
+            for (int k = 1; k < D; ++k) {
+                va += a.vel[k] * nv[k];
+                vb += b.vel[k] * nv[k];
+            }
+            pa = a.p * va;
+            pb = b.p * vb;
+        } else {
+            pa = a.p * a.vel[K];
+            pb = b.p * b.vel[K];
+        }
+        const double pw = pa + pb;
+        f[D + 1] -= 0.5 * pw;
+    }
+}
+
+// Kennedy-Gruber and Ismail-Roe of two cached nodes through the generic evaluation of
+// dg_physics.hpp (CV: contracted with nv).
+template <int D, int K, bool CV>
+__device__ __forceinline__ void other_flux64(const NodeC<double, D> &a, const NodeC<double, D> &b, const double *nv,
+                                             const PhysConst &pc, double *f)
+{
+    Prim<double, D> qa, qb;
+    double ua[D + 2], ub[D + 2];
+    qa.rho = ua[0] = a.u[0];
+    qb.rho = ub[0] = b.u[0];
+    for (int k = 0; k < D; ++k) {
+        qa.vel[k] = a.vel[k];
+        qb.vel[k] = b.vel[k];
+        ua[1 + k] = a.u[0] * a.vel[k];
+        ub[1 + k] = b.u[0] * b.vel[k];
+    }
+    qa.p = a.p;
+    qb.p = b.p;
+    ua[D + 1] = a.u[0] * a.h - a.p;
+    ub[D + 1] = b.u[0] * b.h - b.p;
+    if constexpr (CV) two_point_flux_vec<double, D>(ua, qa, ub, qb, nv, pc, f);
+    else two_point_flux_dir<double, D>(ua, qa, ub, qb, K, pc, f);
+}
+
 // Two-point flux of two cached nodes; Kennedy-Gruber and Ismail-Roe go through
 // the generic evaluation of dg_physics.hpp.
 template <typename T, int D, int K>
 __device__ __forceinline__ void pair_flux_fast(const NodeC<T, D> &a, const NodeC<T, D> &b, const FastConst<T> &fc,
                                                const PhysConst &pc, T *f)
 {
+    if constexpr (std::is_same<T, double>::value) {
+        if (fc.two_point >= 2) ec_flux64<D, K, false>(a, b, nullptr, fc, f);
+        else other_flux64<D, K, false>(a, b, nullptr, pc, f);
+        return;
+    }
     if (fc.two_point >= 2) {
         ec_flux_fast<T, D, K>(a.u[0], a.vel, a.p, a.b, a.v2, b.u[0], b.vel, b.p, b.b, b.v2, fc, f);
     } else {
@@ -213,12 +369,142 @@ __device__ __forceinline__ void roe_fast(const NodeC<T, D> &L, const NodeC<T, D>
     for (int s = 0; s < D + 2; ++s) out[s] = T(-0.5) * A[s];
 }
 
+// Roe-Pike dissipation with Harten's entropy fix in double, -1/2 of it added to out: along the unit
+// normal n (CV) or sgn e_K.  co0 + co3 and (co3 - co0) c are formed once and shared by every state.
+template <int D, int K, bool CV>
+__device__ __forceinline__ void roe64(const NodeC<double, D> &L, const NodeC<double, D> &R, double sgn,
+                                      const double *n, double vnL, double vnR, const FastConst<double> &fc,
+                                      double *out)
+{
+    const double isum = frcp<double>(L.sr + R.sr);
+    const double wL = L.sr * isum, wR = R.sr * isum, rho = L.sr * R.sr;
+    double v[D], v2 = 0.0, vn = 0.0;
+    for (int k = 0; k < D; ++k) {
+        const double a = wL * L.vel[k], b = wR * R.vel[k];
+        v[k] = a + b;
+    }
+    v2 = v[0] * v[0];
+    for (int k = 1; k < D; ++k) v2 += v[k] * v[k];
+    if constexpr (CV) {
+        vn = v[0] * n[0];
+        for (int k = 1; k < D; ++k) vn += v[k] * n[k];
+    } else {
+        vn = v[K] * sgn;
+    }
+    const double ha = wL * L.h, hb = wR * R.h;
+    const double h = ha + hb;
+    const double c2 = fc.gamm1 * (h - 0.5 * v2);
+    double c, ic;
+    Fast<double>::sqrt_rsqrt(c2, &c, &ic);
+    double hic2 = 0.5 * (ic * ic);
+    if (__builtin_expect(!(c2 > 0.0), 0)) {
+        c = 1e10;
+        hic2 = 0.5 * frcp<double>(c2);
+    }
+    double eig[3] = {fab<double>(vn - c), fab<double>(vn), fab<double>(vn + c)};
+    const double eL[3] = {fab<double>(vnL - L.c), fab<double>(vnL), fab<double>(vnL + L.c)};
+    const double eR[3] = {fab<double>(vnR - R.c), fab<double>(vnR), fab<double>(vnR + R.c)};
+    for (int e = 0; e < 3; ++e) {
+        const double eps = fmx<double>(fab<double>(eig[e] - eL[e]), fab<double>(eR[e] - eig[e]));
+        if (eig[e] < eps) eig[e] = 0.5 * (eig[e] * eig[e] * frcp<double>(eps) + eps);
+    }
+    const double dp = R.p - L.p, drho = R.u[0] - L.u[0], dVn = vnR - vnL;
+    const double rc = rho * c * dVn;
+    const double e0 = eig[0] * hic2, e2 = eig[2] * hic2;
+    const double co0 = e0 * (dp - rc), co3 = e2 * (dp + rc);
+    const double s = co0 + co3, dc = (co3 - co0) * c;
+    const double co1 = eig[1] * (drho - 2.0 * dp * hic2), co2 = eig[1] * rho;
+    const double A0 = s + co1;
+    out[0] -= 0.5 * A0;
+    double vt = 0.0;
+    for (int k = 0; k < D; ++k) {
+        double dvt = R.vel[k] - L.vel[k], Ak;
+        if constexpr (CV) {
+            dvt -= dVn * n[k];
+            Ak = A0 * v[k] + co2 * dvt;
+            Ak += dc * n[k];
+        } else {
+            // the normal component of the tangential jump cancels exactly
+            Ak = A0 * v[k];
+            if (k == K) Ak += dc * sgn;
+            else Ak += co2 * dvt;
+        }
+        if (CV || k != K) vt += v[k] * dvt;
+        out[1 + k] -= 0.5 * Ak;
+    }
+    double AE = s * h + dc * vn;
+    AE += co1 * 0.5 * v2;
+    AE += co2 * vt;
+    out[D + 1] -= 0.5 * AE;
+}
+
+// Numerical flux in double along the unit normal n (CV) or sgn e_K, outward of side L; exchanging
+// the sides and turning the normal around gives the exact negative.  GEN: the two-point flux is
+// Kennedy-Gruber or Ismail-Roe, else Chandrashekar or Ranocha; `first` orders the sides for the
+// former, which are not written that way.
+template <int D, int K, bool CV, bool GEN>
+__device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const NodeC<double, D> &R, double sgn,
+                                           const double *n, bool first, const FastConst<double> &fc,
+                                           const PhysConst &pc, double *out)
+{
+    const int cf = fc.conv_flux;
+    double vnL, vnR;
+    if constexpr (CV) {
+        vnL = L.vel[0] * n[0];
+        vnR = R.vel[0] * n[0];
+        for (int k = 1; k < D; ++k) {
+            vnL += L.vel[k] * n[k];
+            vnR += R.vel[k] * n[k];
+        }
+    } else {
+        vnL = L.vel[K] * sgn;
+        vnR = R.vel[K] * sgn;
+    }
+    if (cf >= 3) {
+        if constexpr (!GEN) {
+            ec_flux64<D, K, CV>(L, R, n, fc, out);
+        } else {
+            if (first) other_flux64<D, K, CV>(L, R, n, pc, out);
+            else other_flux64<D, K, CV>(R, L, n, pc, out);
+        }
+        if constexpr (!CV)
+            for (int s = 0; s < D + 2; ++s) out[s] *= sgn;
+    } else {
+        const double mL = L.u[0] * vnL, mR = R.u[0] * vnR, ps = 0.5 * (L.p + R.p);
+        out[0] = 0.5 * (mL + mR);
+        for (int k = 0; k < D; ++k) {
+            const double a = mL * L.vel[k], b = mR * R.vel[k];
+            out[1 + k] = 0.5 * (a + b);
+            if constexpr (CV) out[1 + k] += ps * n[k];
+            else if (k == K) out[1 + k] += ps * sgn;
+        }
+        const double a = mL * L.h, b = mR * R.h;
+        out[D + 1] = 0.5 * (a + b);
+    }
+    if (cf == 0 || cf == 4) {
+        const double hl = 0.5 * fmx<double>(fab<double>(vnL) + L.c, fab<double>(vnR) + R.c);
+        out[0] -= hl * (R.u[0] - L.u[0]);
+        for (int k = 0; k < D; ++k) {
+            const double a = L.u[0] * L.vel[k], b = R.u[0] * R.vel[k];
+            out[1 + k] -= hl * (b - a);
+        }
+        const double a = L.u[0] * L.h - L.p, b = R.u[0] * R.h - R.p;
+        out[D + 1] -= hl * (b - a);
+    }
+    if (cf == 1 || cf == 5) roe64<D, K, CV>(L, R, sgn, n, vnL, vnR, fc, out);
+}
+
 // Numerical flux of a face node along the normal sgn * e_K, L the interior
 // (owner) side.
 template <typename T, int D, int K>
 __device__ __forceinline__ void num_flux_fast(const NodeC<T, D> &L, const NodeC<T, D> &R, T sgn,
                                               const FastConst<T> &fc, const PhysConst &pc, T *out)
 {
+    if constexpr (std::is_same<T, double>::value) {
+        if (fc.two_point >= 2) num_flux64<D, K, false, false>(L, R, sgn, nullptr, true, fc, pc, out);
+        else num_flux64<D, K, false, true>(L, R, sgn, nullptr, true, fc, pc, out);
+        return;
+    }
     const int cf = fc.conv_flux;
     T base[D + 2];
     if (cf >= 3) {
@@ -238,6 +524,80 @@ __device__ __forceinline__ void num_flux_fast(const NodeC<T, D> &L, const NodeC<
     }
     if (cf == 1 || cf == 5) roe_fast<T, D, K>(L, R, sgn, fc, diss);
     for (int s = 0; s < D + 2; ++s) out[s] = base[s] + diss[s];
+}
+
+// ---- Navier-Stokes in double ------------------------------------------------------------------
+// Viscous fluxes of one node in every direction, momentum and energy components only (the density
+// component is zero): f[k][a] = F_v(u, grad u) . e_k, a = 0..D-1 momentum, D energy, the formulas of
+// viscous_flux_all with one reciprocal, 1/rho.
+__device__ __forceinline__ double visc_mu64(const PhysConst &pc, double T_)
+{
+    if (pc.use_constant_viscosity) return pc.mu_const / pc.reynolds;
+    const double tr = pc.temperature_ratio;
+    return (1.0 + tr) * frcp<double>(T_ + tr) * (T_ * fsqrt<double>(T_)) / pc.reynolds;
+}
+
+template <int D>
+__device__ __forceinline__ void viscous_flux64(const double *u, const double *g, const PhysConst &pc,
+                                               double (&f)[D][D + 1])
+{
+    const double gm2 = pc.gam * pc.mach2;
+    const double ir = frcp<double>(u[0]);
+    double vel[D], v2 = 0.0;
+    for (int k = 0; k < D; ++k) {
+        vel[k] = u[1 + k] * ir;
+        v2 += vel[k] * vel[k];
+    }
+    const double T_ = gm2 * pc.gamm1 * (u[D + 1] * ir - 0.5 * v2);
+    const double mu = visc_mu64(pc, T_);
+    const double kappa = mu / (pc.gamm1 * pc.mach2 * pc.prandtl);
+    double vg[D][D], div = 0.0;
+    for (int a = 0; a < D; ++a)
+        for (int b = 0; b < D; ++b) vg[a][b] = (g[(1 + a) * D + b] - vel[a] * g[b]) * ir;
+    for (int a = 0; a < D; ++a) div += vg[a][a];
+    div *= (2.0 / 3.0) * mu;
+    for (int k = 0; k < D; ++k) {
+        // grad p = (gamma - 1) (grad E - v . grad m + |v|^2/2 grad rho)
+        double pg = g[(D + 1) * D + k] + 0.5 * v2 * g[k];
+        for (int a = 0; a < D; ++a) pg -= vel[a] * g[(1 + a) * D + k];
+        const double dT = (gm2 * pc.gamm1 * pg - T_ * g[k]) * ir;
+        double fe = -kappa * dT;
+        for (int a = 0; a < D; ++a) {
+            double tau = mu * (vg[a][k] + vg[k][a]);
+            if (a == k) tau -= div;
+            f[k][a] = -tau;
+            fe -= vel[a] * tau;
+        }
+        f[k][D] = fe;
+    }
+}
+
+// F_v(u, du n) . n for a unit normal n and a state jump du (the SIPG penalty flux): with the
+// gradient du n the velocity gradient is w n, w = (dm - v drho)/rho.
+template <int D>
+__device__ __forceinline__ void viscous_jump64(const NodeC<double, D> &q, const double *du, const double *n,
+                                               const PhysConst &pc, double *f)
+{
+    const double gm2 = pc.gam * pc.mach2;
+    const double ir = frcp<double>(q.u[0]);
+    const double T_ = gm2 * q.p * ir;
+    const double mu = visc_mu64(pc, T_);
+    const double kappa = mu / (pc.gamm1 * pc.mach2 * pc.prandtl);
+    double w[D], wn = 0.0, v2 = 0.0, pg = du[D + 1];
+    for (int k = 0; k < D; ++k) {
+        w[k] = (du[1 + k] - q.vel[k] * du[0]) * ir;
+        wn += w[k] * n[k];
+        v2 += q.vel[k] * q.vel[k];
+        pg -= q.vel[k] * du[1 + k];
+    }
+    pg += 0.5 * v2 * du[0];
+    double fe = -kappa * ((gm2 * pc.gamm1 * pg - T_ * du[0]) * ir);
+    for (int k = 0; k < D; ++k) {
+        const double tau = mu * (w[k] + (1.0 / 3.0) * wn * n[k]);
+        f[k] = -tau;
+        fe -= q.vel[k] * tau;
+    }
+    f[D] = fe;
 }
 
 } // namespace dgx

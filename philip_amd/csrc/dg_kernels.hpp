@@ -188,10 +188,12 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &
             if (a.s4) a.s4[idx] = (a.lsrk_first ? s1 : a.s4[idx]) + a.bhat * r;
         }
     } else {
+        const bool pf_b = std::is_same<T, double>::value && use_pf;
         for (int s = 0; s < NS; ++s) {
             const long idx = base + s * NP;
             const double kk = dudt[s];
-            double accv = a.first_stage ? (a.acc_zero ? 0.0 : a.u0[idx]) : a.acc[idx];
+            // FP64 line kernels: the accumulator and u_n already loaded by the caller into pf2 / pf3
+            double accv = pf_b ? pf2[s] : (a.first_stage ? (a.acc_zero ? 0.0 : a.u0[idx]) : a.acc[idx]);
             accv += a.b_dt * kk;
             a.acc_out[idx] = accv;
             if (a.k_store) a.k_store[idx] = kk;
@@ -205,7 +207,7 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &
                 }
                 if (a_cur != 0.0) st += a_cur * kk;
                 st *= a.dt;
-                st += 1.0 * a.u0[idx];
+                st += 1.0 * (pf_b ? pf3[s] : a.u0[idx]);
                 a.u_next[idx] = st;
             }
         }

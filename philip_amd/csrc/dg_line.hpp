@@ -57,8 +57,9 @@ template <int D, int N, typename T, int ES = 1, bool V = false, bool XJ = false>
     static constexpr int NP = G::NP, NS = D + 2, NL = G::NL;
     static constexpr int EPB = ES > 0 ? G::EPB * ES : (G::EPB / -ES > 0 ? G::EPB / -ES : 1);
     static constexpr bool FAST = std::is_same<T, float>::value;
-    // node cache fields: rho, E, vel[D], p, b, |v|^2, sqrt(rho), c, h
-    static constexpr int NQ = D + 8;
+    // node cache fields: rho, E, vel[D], p, b, |v|^2, sqrt(rho), c, h; FP64: without E (rho h - p)
+    // and |v|^2
+    static constexpr int NQ = FAST ? D + 8 : D + 6;
     // element strides padded to 1 mod 32 words so the stride-N lines of
     // neighbouring elements fall in different LDS banks
     static constexpr int pad1(int x) { return x + (33 - x % 32) % 32; }
@@ -79,11 +80,13 @@ template <int D, int N, typename T, int ES = 1, bool V = false, bool XJ = false>
     static constexpr int ESQ = (QSKEW && FAST) ? pad16(NQ * NP) : (P2D ? pad2d(NQ * NP) : pad1(NQ * NP));
     // Long lines are shared by LS items (the pairs and the viscous columns split evenly), so
     // that the line phase keeps most of the block busy: from p = 4 in 2D and for Navier-Stokes;
-    // for 3D Euler at p = 5, and at p = 6 on the FP64 path only (at p = 4 the extra partials
-    // cost more than the balance gains; at p = 6 the mixed path gained nothing and its batched
-    // kernel's item loop was no longer unrolled, spilling the line sums to scratch)
-    static constexpr int LS = (V || D == 2) ? (N >= 7 ? 3 : (N >= 5 ? 2 : 1))
-                                            : (N >= 7 ? (FAST ? 1 : 3) : (N >= 6 ? 2 : 1));
+    // for 3D Euler at p = 5 (at p = 4 the extra partials cost more than the balance gains; at p = 6
+    // the mixed path gained nothing and its batched kernel's item loop was no longer unrolled,
+    // spilling the line sums to scratch).  FP64 in 3D: 2 items from p = 5, so that one item per
+    // thread holds the sums of one line (at p = 6 three items made 441 of them for 384 threads).
+    static constexpr int LS = (D == 3 && !FAST) ? (N >= 6 ? 2 : 1)
+                              : (V || D == 2)   ? (N >= 7 ? 3 : (N >= 5 ? 2 : 1))
+                                                : (N >= 7 ? 1 : (N >= 6 ? 2 : 1));
     static constexpr int ESV = P2D ? pad2d(LS * NS * NP) : pad1(LS * NS * NP);   // line partials [part][state][node]
     static constexpr int NFN = 2 * D * NL;           // face nodes per element
     // neighbour traces' states [state][face][face node]; each slot then takes that face node's
@@ -94,12 +97,12 @@ template <int D, int N, typename T, int ES = 1, bool V = false, bool XJ = false>
     static constexpr int round64(int x) { return ((x + 63) / 64) * 64; }
     static constexpr int BLOCK = XJ ? round64(EPB * NP > ITEMS + FITEMS ? EPB * NP : ITEMS + FITEMS)
                                     : round64(EPB * NP);
-    // Navier-Stokes (V, mixed path only): own viscous flux in every direction
-    // [direction][state][node] and the neighbours' viscous flux along the face direction at
-    // their face nodes [state][face][face node]
-    static_assert(!V || FAST, "the Navier-Stokes line kernel is the mixed-precision path");
-    static constexpr int ESFV = V ? pad1(D * NS * NP) : 0;
-    static constexpr int ESNV = V ? pad1(NS * NFN) : 0;
+    // Navier-Stokes (V): own viscous flux in every direction [direction][state][node] and the
+    // neighbours' viscous flux along the face direction at their face nodes
+    // [state][face][face node]; FP64 leaves out the density component, which is zero
+    static constexpr int NVS = FAST ? NS : D + 1;
+    static constexpr int ESFV = V ? pad1(D * NVS * NP) : 0;
+    static constexpr int ESNV = V ? pad1(NVS * NFN) : 0;
     static constexpr int EIN = ESQ + ESN + ESFV + ESNV;
     // [traces / surface terms | node cache | V: viscous fluxes]; the line partials take the node
     // cache's place (and what follows it) once every item has run
@@ -147,6 +150,16 @@ template <int D, int N> __device__ __forceinline__ int qpos(int i)
 template <typename T, int D>
 __device__ __forceinline__ void nodef_store(T *q, int st, const NodeC<T, D> &n)
 {
+    if constexpr (std::is_same<T, double>::value) {
+        q[0] = n.u[0];
+        for (int k = 0; k < D; ++k) q[(1 + k) * st] = n.vel[k];
+        q[(D + 1) * st] = n.p;
+        q[(D + 2) * st] = n.b;
+        q[(D + 3) * st] = n.h;
+        q[(D + 4) * st] = n.c;
+        q[(D + 5) * st] = n.sr;
+        return;
+    }
     q[0] = n.u[0];
     q[st] = n.u[D + 1];
     for (int k = 0; k < D; ++k) q[(2 + k) * st] = n.vel[k];
@@ -163,9 +176,25 @@ template <typename T, int D> __device__ __forceinline__ void node_canon(NodeC<T,
     for (int k = 0; k < D; ++k) n.u[1 + k] = n.u[0] * n.vel[k];
 }
 
+// FP64: the fields of a two-point flux (rho, v, p, b), and all of them for a surface flux.
+template <int D> __device__ __forceinline__ void nodef_load_pair(const double *q, int st, NodeC<double, D> &n)
+{
+    n.u[0] = q[0];
+    for (int k = 0; k < D; ++k) n.vel[k] = q[(1 + k) * st];
+    n.p = q[(D + 1) * st];
+    n.b = q[(D + 2) * st];
+}
+
 template <typename T, int D>
 __device__ __forceinline__ void nodef_load(const T *q, int st, NodeC<T, D> &n)
 {
+    if constexpr (std::is_same<T, double>::value) {
+        nodef_load_pair<D>(q, st, n);
+        n.h = q[(D + 3) * st];
+        n.c = q[(D + 4) * st];
+        n.sr = q[(D + 5) * st];
+        return;
+    }
     n.u[0] = q[0];
     n.u[D + 1] = q[st];
     for (int k = 0; k < D; ++k) n.vel[k] = q[(2 + k) * st];
@@ -226,6 +255,46 @@ template <int N, int LS, int H> __device__ __forceinline__ constexpr bool pair_i
     return idx >= H * NPAIR / LS && idx < (H + 1) * NPAIR / LS;
 }
 
+// FP64: two-point fluxes of part H of a line with the two-point flux TP (2 Chandrashekar, 3 Ranocha,
+// 0 the generic evaluation; a constant, so that an item's code holds one of them and loads what it
+// needs).  CV: contracted with the pair's average cofactor column, cm the nodes' columns.
+template <int D, int N, int K, int LS, int H, bool CV, int TP>
+__device__ __forceinline__ void pairs64(const Ops1D &ops, const PhysConst &pc, const FastConst<double> &fc0,
+                                        const double *sq, const double (&cm)[CV ? N : 1][D], int line,
+                                        double (&acc)[N][D + 2])
+{
+    constexpr int NP = Geo<D, N>::NP, NS = D + 2;
+    FastConst<double> fc = fc0;
+    if (TP) fc.two_point = TP;
+#pragma unroll
+    for (int p0 = 0; p0 < N; ++p0) {
+#pragma unroll
+        for (int p1 = p0 + 1; p1 < N; ++p1) {
+            if (!pair_in_part<N, LS, H>(p0, p1)) continue;
+            NodeC<double, D> A, B;
+            nodef_load_pair<D>(sq + qpos<D, N>(line_node<D, N>(K, line, p0)), NP, A);
+            nodef_load_pair<D>(sq + qpos<D, N>(line_node<D, N>(K, line, p1)), NP, B);
+            double nv[D], F[NS];
+            if constexpr (CV)
+                for (int m = 0; m < D; ++m) nv[m] = 0.5 * (cm[p0][m] + cm[p1][m]);
+            if constexpr (TP > 0) {
+                ec_flux64<D, K, CV>(A, B, nv, fc, F);
+            } else {
+                const double *qa = sq + qpos<D, N>(line_node<D, N>(K, line, p0)) + (D + 3) * NP;
+                const double *qb = sq + qpos<D, N>(line_node<D, N>(K, line, p1)) + (D + 3) * NP;
+                A.h = qa[0];
+                B.h = qb[0];
+                other_flux64<D, K, CV>(A, B, nv, pc, F);
+            }
+            const double s01 = ops.Sk[p0][p1], s10 = ops.Sk[p1][p0];
+            for (int s = 0; s < NS; ++s) {
+                acc[p0][s] -= s01 * F[s];
+                acc[p1][s] -= s10 * F[s];
+            }
+        }
+    }
+}
+
 template <typename T, int D, int N, int K, int LS = 1, int H = 0>
 __device__ __forceinline__ void pairs_f(const Ops1D &ops, const PhysConst &pc, const FastConst<T> &fc, const T *sq,
                                         int line, T (&acc)[N][D + 2])
@@ -271,6 +340,33 @@ __device__ __forceinline__ void visc_line(const Ops1D &ops, const T *sfv, int li
         for (int a2 = 0; a2 < N; ++a2) {
             const T dab = op_d<T>(ops, a2, b);
             for (int s = 0; s < NS; ++s) acc[a2][s] -= dab * fv[s];
+        }
+    }
+}
+
+// The same in double, momentum and energy components of the physical fluxes [direction][state][node]
+// (CV: contracted with the node's cofactor column cm).
+template <int D, int N, int K, int LS, int H, bool CV>
+__device__ __forceinline__ void visc_line64(const Ops1D &ops, const double *sfv, const double (&cm)[CV ? N : 1][D],
+                                            int line, double (&acc)[N][D + 2])
+{
+    constexpr int NP = Geo<D, N>::NP, NVS = D + 1;
+#pragma unroll
+    for (int b = H * N / LS; b < (H + 1) * N / LS; ++b) {
+        const int nb = line_node<D, N>(K, line, b);
+        double fv[NVS];
+        for (int s = 0; s < NVS; ++s) {
+            if constexpr (CV) {
+                fv[s] = sfv[s * NP + nb] * cm[b][0];
+                for (int m = 1; m < D; ++m) fv[s] += sfv[(m * NVS + s) * NP + nb] * cm[b][m];
+            } else {
+                fv[s] = sfv[(K * NVS + s) * NP + nb];
+            }
+        }
+#pragma unroll
+        for (int a2 = 0; a2 < N; ++a2) {
+            const double dab = ops.D[a2][b];
+            for (int s = 0; s < NVS; ++s) acc[a2][1 + s] -= dab * fv[s];
         }
     }
 }
@@ -323,25 +419,10 @@ __device__ __forceinline__ void face_f(const Ops1D &ops, const PhysConst &pc, co
     const int fj = line_node<D, N>(K, fn, side ? 0 : N - 1);
     NodeC<T, D> qi, qn, L, R;
     nodef_load<T, D>(in.sq + le * LG::ESQ + qpos<D, N>(fi), NP, qi);
-    bool own = e < nb;
-    if constexpr (BND) {
-        if (nb < 0) {
-            // boundary face of type -nb: the exterior state from the interior node
-            T ub[NS];
-            boundary_state<T, D>(-nb, qi.u, K, side ? T(1) : T(-1), pc, ub);
-            for (int s = 0; s < NS; ++s) qn.u[s] = ub[s];
-            node_fill<T, D>(qn, fc);
-            node_canon<T, D>(qn);
-            own = true;
-        } else if (nbl >= 0) {
-            nodef_load<T, D>(in.sq + nbl * LG::ESQ + qpos<D, N>(fj), NP, qn);
-        } else {
-            trace_node<T, D>(in.tr, in.tst, fc, qn);
-        }
-    } else {
-        if (nbl >= 0) nodef_load<T, D>(in.sq + nbl * LG::ESQ + qpos<D, N>(fj), NP, qn);
-        else trace_node<T, D>(in.tr, in.tst, fc, qn);
-    }
+    // a boundary face's interior is its cell; its trace is the exterior state
+    const bool own = e < nb || (BND && nb < 0);
+    if (nbl >= 0) nodef_load<T, D>(in.sq + nbl * LG::ESQ + qpos<D, N>(fj), NP, qn);
+    else trace_node<T, D>(in.tr, in.tst, fc, qn);
     nodef_select<T, D>(own, qi, qn, L);
     nodef_select<T, D>(own, qn, qi, R);
     const T sgn = side ? T(1) : T(-1);
@@ -372,15 +453,129 @@ __device__ __forceinline__ void face_f(const Ops1D &ops, const PhysConst &pc, co
     }
 }
 
+// Surface term in double, the flux along the element's outward normal; num_flux64 gives the exact
+// negative from the other side, so neither the owner rule nor the block that evaluates a face
+// changes its bits.  CV: along the physical normal C n_ref of the face's owner (the lower cell
+// index), scaled by its length.  trv (V): the neighbour's viscous flux along e_K, or (CV)
+// contracted with the owner's cofactor column.
+template <int D, int N, int K, bool V, bool CV, bool BND, bool GEN>
+__device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, const PhysConst &pc,
+                                       const FastConst<double> &fc, const FaceIn<double> &in, int le, int side, int fn,
+                                       int e, int nb, int nbl, double (&out)[D + 2], double (&out_nb)[D + 2])
+{
+    using LG = LineGeo<D, N, double, 1, V>;
+    constexpr int NP = LG::NP, NS = D + 2, NVS = LG::NVS, MS = D * D + 1;
+    const int fi = line_node<D, N>(K, fn, side ? N - 1 : 0);
+    const int fj = line_node<D, N>(K, fn, side ? 0 : N - 1);
+    const bool own = e < nb || (BND && nb < 0);
+    const double sgn = side ? 1.0 : -1.0;
+    double nc[D], nh[D], area = 1.0;  // CV: owner's column, unit outward normal, area
+    if constexpr (CV) {
+        const double *c = a.met + (own ? (long)e * MS * NP + fi : (long)nb * MS * NP + fj);
+        double a2 = 0.0;
+        for (int m = 0; m < D; ++m) {
+            nc[m] = c[(m * D + K) * NP];
+            a2 += nc[m] * nc[m];
+        }
+        double ia;
+        Fast<double>::sqrt_rsqrt(a2, &area, &ia);
+        for (int m = 0; m < D; ++m) nh[m] = (sgn * nc[m]) * ia;
+    } else {
+        for (int m = 0; m < D; ++m) nh[m] = (m == K) ? sgn : 0.0;
+    }
+    NodeC<double, D> qi, qn;
+    nodef_load<double, D>(in.sq + le * LG::ESQ + qpos<D, N>(fi), NP, qi);
+    if (nbl >= 0) {
+        nodef_load<double, D>(in.sq + nbl * LG::ESQ + qpos<D, N>(fj), NP, qn);
+    } else {
+        for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
+        node_fill<double, D>(qn, fc);
+    }
+    double fs[NS];
+    num_flux64<D, K, CV, GEN>(qi, qn, sgn, nh, own, fc, pc, fs);
+    const double iwb = ops.inv_wb;
+    const double w = CV ? iwb * area : iwb;
+    for (int s = 0; s < NS; ++s) {
+        out[s] = -(w * fs[s]);
+        out_nb[s] = -out[s];
+    }
+    if constexpr (V) {
+        // average of the one-sided viscous fluxes (antisymmetric between the sides) and, one-sided,
+        // the strong form's interior flux
+        const double *va = in.sfv + le * LG::ESFV + fi, *vb = in.sfv + (nbl >= 0 ? nbl : 0) * LG::ESFV + fj;
+        double fa[NVS], fb[NVS], ia[NVS], ib[NVS];
+        if constexpr (CV) {
+            const double *ca = a.met + (long)e * MS * NP + fi, *cb = a.met + (long)nb * MS * NP + fj;
+            for (int s = 0; s < NVS; ++s) {
+                fa[s] = ia[s] = fb[s] = ib[s] = 0.0;
+                for (int m = 0; m < D; ++m) {
+                    const double p = va[(m * NVS + s) * NP];
+                    fa[s] += p * nc[m];
+                    ia[s] += p * ca[(m * D + K) * NP];
+                }
+                if (nbl >= 0) {
+                    for (int m = 0; m < D; ++m) {
+                        const double p = vb[(m * NVS + s) * NP];
+                        fb[s] += p * nc[m];
+                        ib[s] += p * cb[(m * D + K) * NP];
+                    }
+                } else {
+                    fb[s] = in.trv[s * in.tst];
+                }
+            }
+        } else {
+            for (int s = 0; s < NVS; ++s) {
+                fa[s] = va[(K * NVS + s) * NP];
+                fb[s] = (nbl >= 0) ? vb[(K * NVS + s) * NP] : in.trv[s * in.tst];
+                ia[s] = fa[s];
+                ib[s] = fb[s];
+            }
+        }
+        double pj[NVS];
+        for (int s = 0; s < NVS; ++s) pj[s] = 0.0;
+        if (pc.diss_flux == 0) {
+            double du[NS], ja[NVS], jb[NVS];
+            du[0] = qi.u[0] - qn.u[0];
+            for (int k = 0; k < D; ++k) {
+                const double ma = qi.u[0] * qi.vel[k], mb = qn.u[0] * qn.vel[k];
+                du[1 + k] = ma - mb;
+            }
+            const double ea = qi.u[0] * qi.h - qi.p, eb = qn.u[0] * qn.h - qn.p;
+            du[D + 1] = ea - eb;
+            viscous_jump64<D>(qi, du, nh, pc, ja);
+            viscous_jump64<D>(qn, du, nh, pc, jb);
+            double pen = a.penalty;
+            if constexpr (CV) pen = 0.5 * (a.pen[(long)e * D + K] + a.pen[(long)nb * D + K]) * area;
+            for (int s = 0; s < NVS; ++s) {
+                const double js = ja[s] + jb[s];
+                pj[s] = 0.5 * pen * js;
+            }
+        }
+        for (int s = 0; s < NVS; ++s) {
+            const double av = fa[s] + fb[s];
+            const double fvs = 0.5 * sgn * av - pj[s];
+            out[1 + s] += iwb * (sgn * ia[s] - fvs);
+            out_nb[1 + s] += iwb * (fvs - sgn * ib[s]);
+        }
+    }
+}
+
 // One block's work: elements blk0 .. blk0 + EPB - 1 of the solve described by a.
 // V: Navier-Stokes (split convective form plus the viscous volume and surface
 // terms, with the lifted gradient a.aux computed beforehand).
-template <int D, int N, typename T, int ES, bool V = false, bool XJ = false, bool BND = false>
+// CV (FP64): curvilinear grid, metric terms a.met.  BND: Euler boundary faces.  GEN (FP64): the
+// two-point flux is Kennedy-Gruber or Ismail-Roe, else Chandrashekar or Ranocha: a kernel of its own,
+// since the generic evaluation sets the register count of a kernel that holds both (p=3: 153 VGPRs,
+// the curved kernel 246).
+template <int D, int N, typename T, int ES, bool V = false, bool XJ = false, bool BND = false, bool CV = false,
+          bool GEN = false>
 __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops, const PhysConst &pc, const int blk0)
 {
     using LG = LineGeo<D, N, T, ES, V, XJ>;
     constexpr int NP = LG::NP, NS = LG::NS, NL = LG::NL, EPB = LG::EPB, BLOCK = LG::BLOCK, LS = LG::LS;
     constexpr bool FAST = LG::FAST;
+    static_assert(!(CV && FAST) && !(BND && (V || CV)), "no such line kernel");
+    constexpr int MS = D * D + 1;             // metric slots per node in a.met
     constexpr int NFI = (LG::FITEMS + BLOCK - 1) / BLOCK;  // face-trace loads per thread
     constexpr int NFS = EPB * 2 * D;                       // face sides of the block
     constexpr int NWAVE = BLOCK / 64;
@@ -443,6 +638,11 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
                     const int fj = line_node<D, N>(f >> 1, fn, (f & 1) ? 0 : N - 1);
                     for (int s = 0; s < NS; ++s) un[j][s] = a.u[((long)nb * NS + s) * NP + fj];
                     fdst[j] = t;  // = fle * NFN + r
+                } else if (BND && nb < 0) {
+                    // boundary face: its trace is the exterior state, from the interior one
+                    const int fi = line_node<D, N>(f >> 1, fn, (f & 1) ? N - 1 : 0);
+                    for (int s = 0; s < NS; ++s) un[j][s] = a.u[((long)fe * NS + s) * NP + fi];
+                    fdst[j] = t;
                 }
             }
         }
@@ -458,9 +658,69 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
     for (int j = 0; j < NFI; ++j) {
         if (fdst[j] < 0) continue;
         T *q = sN + (fdst[j] / LG::NFN) * LG::ESN + fdst[j] % LG::NFN;
+        if constexpr (BND) {
+            if (nbv[j] < 0) {
+                // evaluated here, where few values are live, and not among the face items: there
+                // its powers and branches had the FP64 kernel spill 416 B/lane at p=4
+                const int f = (fdst[j] % LG::NFN) / NL;
+                NodeC<T, D> n;
+                for (int s = 0; s < NS; ++s) n.u[s] = T(un[j][s]);
+                if constexpr (FAST) {
+                    node_fill<T, D>(n, fc);
+                    node_canon<T, D>(n);
+                }
+                T ub[NS];
+                boundary_state<T, D>(-nbv[j], n.u, f >> 1, (f & 1) ? T(1) : T(-1), pc, ub);
+                for (int s = 0; s < NS; ++s) q[s * LG::NFN] = ub[s];
+                continue;
+            }
+        }
         for (int s = 0; s < NS; ++s) q[s * LG::NFN] = T(un[j][s]);
     }
-    if constexpr (V) {
+    if constexpr (V && !FAST) {
+        // viscous fluxes from the lifted gradient: the own nodes' physical fluxes, the neighbours'
+        // face nodes' along the face direction (CV: contracted with the owner's column)
+        constexpr int NVS = LG::NVS;
+        if (active) {
+            double g[NS * D], ut[NS], fv[D][NVS];
+#pragma unroll
+            for (int x = 0; x < NS * D; ++x) g[x] = a.aux[x % D][((long)e * NS + x / D) * NP + i];
+            for (int s = 0; s < NS; ++s) ut[s] = ud[s];
+            viscous_flux64<D>(ut, g, pc, fv);
+#pragma unroll
+            for (int k = 0; k < D; ++k)
+                for (int s = 0; s < NVS; ++s) sFv[le * LG::ESFV + (k * NVS + s) * NP + i] = fv[k][s];
+        }
+#pragma unroll
+        for (int j = 0; j < NFI; ++j) {
+            if (fdst[j] < 0) continue;
+            const int t = tid + j * BLOCK;
+            const int f = (t % LG::NFN) / NL, fn = t % NL;
+            const int fj = line_node<D, N>(f >> 1, fn, (f & 1) ? 0 : N - 1);
+            const long nb = nbv[j];
+            double g[NS * D], fv[D][NVS], fk[NVS];
+#pragma unroll
+            for (int x = 0; x < NS * D; ++x) g[x] = a.aux[x % D][(nb * NS + x / D) * NP + fj];
+            viscous_flux64<D>(un[j], g, pc, fv);
+            if constexpr (CV) {
+                const int fe = blk0 + t / LG::NFN;
+                const int fi = line_node<D, N>(f >> 1, fn, (f & 1) ? N - 1 : 0);
+                const double *c = a.met + (fe < nb ? (long)fe * MS * NP + fi : nb * MS * NP + fj) + (f >> 1) * NP;
+                for (int s = 0; s < NVS; ++s) {
+                    fk[s] = fv[0][s] * c[0];
+                    for (int m = 1; m < D; ++m) fk[s] += fv[m][s] * c[m * D * NP];
+                }
+            } else {
+                for (int s = 0; s < NVS; ++s) fk[s] = fv[0][s];
+#pragma unroll
+                for (int k = 1; k < D; ++k)
+                    for (int s = 0; s < NVS; ++s) fk[s] = (f >> 1) == k ? fv[k][s] : fk[s];
+            }
+            for (int s = 0; s < NVS; ++s)
+                sNv[(fdst[j] / LG::NFN) * LG::ESNV + fdst[j] % LG::NFN + s * LG::NFN] = fk[s];
+        }
+    }
+    if constexpr (V && FAST) {
         // viscous fluxes from the lifted gradient: the own nodes' in every direction, the
         // neighbours' face nodes' along the face direction
         if (active) {
@@ -541,8 +801,30 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
             const T *q = sQ + lle * LG::ESQ;
             auto pitem = [&](auto kc, auto hc) {
                 constexpr int K = decltype(kc)::value, H = decltype(hc)::value;
-                pairs_f<T, D, N, K, LS, H>(ops, pc, fc, q, line, rp[j < JP ? j : 0]);
-                if constexpr (V) visc_line<D, N, K, T, LS, H>(ops, sFv + lle * LG::ESFV, line, rp[j < JP ? j : 0]);
+                T(&acc)[N][NS] = rp[j < JP ? j : 0];
+                if constexpr (FAST) {
+                    pairs_f<T, D, N, K, LS, H>(ops, pc, fc, q, line, acc);
+                    if constexpr (V) visc_line<D, N, K, T, LS, H>(ops, sFv + lle * LG::ESFV, line, acc);
+                } else {
+                    double cm[CV ? N : 1][D];
+                    if constexpr (CV) {
+#pragma unroll
+                        for (int p = 0; p < N; ++p)
+                            for (int m = 0; m < D; ++m)
+                                cm[p][m] = a.met[((long)(blk0 + lle) * MS + m * D + K) * NP +
+                                                 line_node<D, N>(K, line, p)];
+                    }
+#pragma unroll
+                    for (int p = 0; p < N; ++p)
+                        for (int s = 0; s < NS; ++s) acc[p][s] = 0.0;
+                    if constexpr (GEN) {
+                        pairs64<D, N, K, LS, H, CV, 0>(ops, pc, fc, q, cm, line, acc);
+                    } else {
+                        if (fc.two_point == 2) pairs64<D, N, K, LS, H, CV, 2>(ops, pc, fc, q, cm, line, acc);
+                        else pairs64<D, N, K, LS, H, CV, 3>(ops, pc, fc, q, cm, line, acc);
+                    }
+                    if constexpr (V) visc_line64<D, N, K, LS, H, CV>(ops, sFv + lle * LG::ESFV, cm, line, acc);
+                }
             };
             auto pdir = [&](auto kc) {
                 if (h == 0) pitem(kc, std::integral_constant<int, 0>{});
@@ -565,7 +847,10 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
             T rf[NS], rfn[NS];
             auto fitem = [&](auto kc) {
                 constexpr int K = decltype(kc)::value;
-                face_f<T, D, N, K, V, BND>(ops, pc, fc, in, fle, side, fn, blk0 + fle, nb, nbl, pen, rf, rfn);
+                if constexpr (FAST)
+                    face_f<T, D, N, K, V, BND>(ops, pc, fc, in, fle, side, fn, blk0 + fle, nb, nbl, pen, rf, rfn);
+                else
+                    face64<D, N, K, V, CV, BND, GEN>(a, ops, pc, fc, in, fle, side, fn, blk0 + fle, nb, nbl, rf, rfn);
             };
             if (k == 0) fitem(std::integral_constant<int, 0>{});
             else if (k == 1) fitem(std::integral_constant<int, 1>{});
@@ -581,7 +866,8 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
     }
     __syncthreads();  // node cache and traces consumed; their storage now takes the partials
     constexpr bool LATE_PF = !PREFETCH && !FAST && line_late_prefetch_d<D, N>();
-    const bool late_pf = LATE_PF && active && a.mode == MODE_LSRK && !a.lsrk_first;
+    const bool late_pf = LATE_PF && active &&
+                         ((a.mode == MODE_LSRK && !a.lsrk_first) || a.mode == MODE_BUTCHER);
     // FP64 at N >= 4: the stage state is read again here for the epilogue (an L2 hit: the block
     // read it in phase A) instead of being held in registers through the line phase (TGV 32^3
     // p=3: 177 -> 170 us per stage, 64 -> 16 B/lane of spills; p=4 24^3 294 -> 244 us; at p=2
@@ -590,12 +876,20 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
     double ue[NS];
     if (REREAD && active && a.mode == MODE_LSRK)
         for (int s = 0; s < NS; ++s) ue[s] = a.u[((long)e * NS + s) * NP + i];
-    if (late_pf)
+    if (late_pf) {
+        // LSRK: S2 and S3; Butcher: the accumulator (u_n at the first stage, nothing for relaxation
+        // RK there) and u_n
+        const bool lsrk = a.mode == MODE_LSRK;
+        const double *p2 = lsrk ? a.s2 : (a.first_stage ? (a.acc_zero ? nullptr : a.u0) : a.acc);
+        const double *p3 = lsrk ? a.s3 : (a.u_next ? a.u0 : nullptr);
         for (int s = 0; s < NS; ++s) {
             const long idx = ((long)e * NS + s) * NP + i;
-            pf2[s] = ld_stream(a.s2 + idx);
-            pf3[s] = ld_stream(a.s3 + idx);
+            pf2[s] = p2 ? ld_stream(p2 + idx) : 0.0;
+            pf3[s] = p3 ? ld_stream(p3 + idx) : 0.0;
         }
+    }
+    double jac = 0.0;
+    if (CV && active) jac = a.met[((long)e * MS + D * D) * NP + i];
     // Line partials of one direction at a time into one [part][state][node] buffer: direction 0
     // stores, each later direction adds after a barrier, so every part's sum is ((d0 + d1) + d2)
     // in this order in every block layout.
@@ -647,8 +941,8 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
         const T *w = fb + f * NL + node_line<D, N>(k, i);
         for (int s = 0; s < NS; ++s) acc[s] += w[s * LG::NFN];
     }
-    if constexpr (REREAD) stage_epilogue<D, N, T>(a, ops, e, i, c, ue, acc, late_pf, pf2, pf3);
-    else stage_epilogue<D, N, T>(a, ops, e, i, c, ud, acc, pf || late_pf, pf2, pf3);
+    if constexpr (REREAD) stage_epilogue<D, N, T>(a, ops, e, i, c, ue, acc, late_pf, pf2, pf3, jac);
+    else stage_epilogue<D, N, T>(a, ops, e, i, c, ud, acc, pf || late_pf, pf2, pf3, jac);
 }
 
 // Elements-per-block variant (ES of LineGeo) of the single-solve Euler line kernel: the mixed path
@@ -663,31 +957,30 @@ template <int D, int N, typename T> using LineGeoS = LineGeo<D, N, T, line_es_si
 
 // One solve: blocks in XCD-aware order over the element groups.  BND: the mesh has boundary
 // faces (a separate instantiation, so the periodic kernels carry no boundary code).
-template <int D, int N, typename T, bool BND = false>
+template <int D, int N, typename T, bool BND = false, bool GEN = false>
 __global__ void __launch_bounds__((LineGeoS<D, N, T>::BLOCK))
 line_kernel(StageArgs a, Ops1D ops, PhysConst pc)
 {
-    line_block<D, N, T, line_es_single<D, N, T>(), false, false, BND>(a, ops, pc,
-                                                                       xcd_block() * LineGeoS<D, N, T>::EPB);
+    line_block<D, N, T, line_es_single<D, N, T>(), false, false, BND, false, GEN>(
+        a, ops, pc, xcd_block() * LineGeoS<D, N, T>::EPB);
 }
 // Waves per SIMD the single-solve 3D line kernel is held to (amdgpu_waves_per_eu; 0: the
 // compiler's choice).  The mixed path keeps the compiler's choice (a 4-wave bound at p=6 was
 // faster with an earlier, larger LDS layout; it now measures 296 against 278 us per stage at 16^3).
-// FP64 path at p=3..5: 3 (168 VGPRs, ~64 B/lane spilled at p=3,
-// two -> three blocks per CU): TGV p=3 32^3 258 -> 222 us per stage, p=4 24^3 327 -> 305 us,
-// p=5 20^3 398 -> 370 us (4 waves at p=3: 395 us); at p=2 no change and at p=6 much slower
-// (448 -> 724 us), so those keep the compiler's choice.
+// FP64 path at p=3..5: 3 (168 VGPRs; p=3 takes 153 and spills nothing, TGV p=3 32^3 140 us per
+// stage); at p=2 no change and at p=6 much slower (448 -> 724 us with an earlier form of the
+// fluxes), so those keep the compiler's choice.
 template <int D, int N, typename T> constexpr int line_waves()
 {
     if constexpr (D == 3 && N >= 4 && N <= 6 && std::is_same<T, double>::value) return 3;
     return 0;
 }
-template <int D, int N, typename T, int W, bool BND = false>
+template <int D, int N, typename T, int W, bool BND = false, bool GEN = false>
 __global__ void __launch_bounds__((LineGeoS<D, N, T>::BLOCK)) __attribute__((amdgpu_waves_per_eu(W)))
 line_kernel_wb(StageArgs a, Ops1D ops, PhysConst pc)
 {
-    line_block<D, N, T, line_es_single<D, N, T>(), false, false, BND>(a, ops, pc,
-                                                                       xcd_block() * LineGeoS<D, N, T>::EPB);
+    line_block<D, N, T, line_es_single<D, N, T>(), false, false, BND, false, GEN>(
+        a, ops, pc, xcd_block() * LineGeoS<D, N, T>::EPB);
 }
 
 // Navier-Stokes, mixed path.  line_kernel_ns_w4 is held to 4 waves/SIMD (128 VGPRs; a few
@@ -714,23 +1007,23 @@ line_kernel_ns_w4(StageArgs a, Ops1D ops, PhysConst pc)
 struct BatchBlock {
     int inst, blk0;
 };
-template <int D, int N, typename T, int ES, bool XJ>
+template <int D, int N, typename T, int ES, bool XJ, bool GEN>
 __global__ void __launch_bounds__((LineGeo<D, N, T, ES, false, XJ>::BLOCK))
 line_kernel_batch(const BatchBlock *__restrict__ blocks, const StageArgs *__restrict__ args,
                   const PhysConst *__restrict__ pcs, Ops1D ops)
 {
     const BatchBlock bb = blocks[xcd_block()];
-    line_block<D, N, T, ES, false, XJ>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
+    line_block<D, N, T, ES, false, XJ, false, false, GEN>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
 }
 // The same held to W waves/SIMD (amdgpu_waves_per_eu): a candidate tile of the batched
 // autotuner.
-template <int D, int N, typename T, int ES, int W, bool XJ>
+template <int D, int N, typename T, int ES, int W, bool XJ, bool GEN>
 __global__ void __launch_bounds__((LineGeo<D, N, T, ES, false, XJ>::BLOCK)) __attribute__((amdgpu_waves_per_eu(W)))
 line_kernel_batch_wb(const BatchBlock *__restrict__ blocks, const StageArgs *__restrict__ args,
                      const PhysConst *__restrict__ pcs, Ops1D ops)
 {
     const BatchBlock bb = blocks[xcd_block()];
-    line_block<D, N, T, ES, false, XJ>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
+    line_block<D, N, T, ES, false, XJ, false, false, GEN>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
 }
 
 // Tiles the batched autotuner times per (dim, nodes per direction, precision): elements per
