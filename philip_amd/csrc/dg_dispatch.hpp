@@ -55,6 +55,27 @@ void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
     const bool split = c->P.use_split_form != 0;
     const bool nsv = c->P.pde == DGX_NAVIER_STOKES;
     const bool bnd = c->has_boundary;
+    if constexpr (std::is_same<T, double>::value) {
+        // FP64 Chandrashekar / Ranocha split form with the viscous terms or on a curvilinear grid, no
+        // boundary faces
+        if (split && !bnd && (nsv || c->curv) && c->pc.two_point >= 2) {
+            auto go = [&](auto vc, auto cc) {
+                constexpr bool V = decltype(vc)::value, CV = decltype(cc)::value;
+                using LV = LineGeoK<D, N, T, V>;
+                hipLaunchKernelGGL((line64_kernel<D, N, V, CV>), dim3((c->ncells + LV::EPB - 1) / LV::EPB),
+                                   dim3(LV::BLOCK), 0, c->stream, a, c->ops, c->pc);
+            };
+            if constexpr (D == 3) {
+                if (nsv) {
+                    if (c->curv) go(std::true_type{}, std::true_type{});
+                    else go(std::true_type{}, std::false_type{});
+                    return;
+                }
+            }
+            go(std::false_type{}, std::true_type{});
+            return;
+        }
+    }
     if (c->curv) {  // curvilinear grid: stage2_kernel with the metric terms, boundaries included
         if constexpr (D == 3) {
             if (nsv) {

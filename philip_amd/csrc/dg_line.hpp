@@ -125,6 +125,7 @@ template <int D, int N, typename T, bool V> constexpr int line_es()
     }
 }
 template <int D, int N, typename T, bool V> using LineGeoK = LineGeo<D, N, T, line_es<D, N, T, V>(), V>;
+template <int D, int N, bool V, bool CV> constexpr int line64_waves() { return 2; }
 
 // ---- node cache in LDS ----------------------------------------------------
 // Position of node i (x fastest) in its element's cache.  3D, N = 4: the skewed order
@@ -981,6 +982,21 @@ line_kernel_wb(StageArgs a, Ops1D ops, PhysConst pc)
 {
     line_block<D, N, T, line_es_single<D, N, T>(), false, false, BND, false, GEN>(
         a, ops, pc, xcd_block() * LineGeoS<D, N, T>::EPB);
+}
+
+// FP64 with the viscous terms (V) and / or on a curvilinear grid (CV), Chandrashekar and Ranocha
+// fluxes.  What stage2_kernel spent on these was VALU issue (IEEE divisions, the viscous flux of a
+// node evaluated per direction, log means by division); the cached-node items need about a third of
+// the instructions.  Right-hand side, stage2_kernel -> here: curved Euler p=3 32^3 400 -> 160 us,
+// curved Navier-Stokes p=5 16^3 611 -> 246 us (with the 66 us lifted gradient), Navier-Stokes
+// p=5 16^3 stage 264 -> 160 us.  The metric columns are read from memory by the one item that uses
+// them, so the block's LDS is that of the box.
+template <int D, int N, bool V, bool CV>
+__global__ void __launch_bounds__((LineGeoK<D, N, double, V>::BLOCK)) __attribute__((amdgpu_waves_per_eu(line64_waves<D, N, V, CV>())))
+line64_kernel(StageArgs a, Ops1D ops, PhysConst pc)
+{
+    line_block<D, N, double, line_es<D, N, double, V>(), V, false, false, CV>(
+        a, ops, pc, xcd_block() * LineGeoK<D, N, double, V>::EPB);
 }
 
 // Navier-Stokes, mixed path.  line_kernel_ns_w4 is held to 4 waves/SIMD (128 VGPRs; a few

@@ -1,6 +1,8 @@
-"""The FP64 line kernel against the oracle where its blocking can go wrong: boundary faces, whose
-exterior states are the traces of its face items, with two cells a side and with cell counts that
-leave a part of the last block empty.  Bar: 1e-12 of the sum of the absolute values of a DoF's terms, as in the other
+"""The FP64 line kernel with the viscous terms and on curvilinear grids (Chandrashekar and Ranocha
+split forms) against the oracle where its blocking can go wrong: two cells a side (a cell is its own
+neighbour's neighbour on both sides), cell counts that leave a part of the last block empty, every
+degree, both viscous numerical fluxes; and boundary faces, whose exterior states are the traces of
+its face items.  Bar: 1e-12 of the sum of the absolute values of a DoF's terms, as in the other
 residual parity tests."""
 import numpy as np
 import pytest
@@ -35,6 +37,27 @@ def check(kw, seed):
 
 
 SPLIT = dict(use_split_form=1, mach_inf=0.3)
+NS = dict(pde=P.NAVIER_STOKES, use_constant_viscosity=0, reynolds_inf=200.0, prandtl=0.71)
+
+
+@pytest.mark.parametrize("p,n", [(1, 2), (1, 5), (2, 3), (3, 2), (3, 3), (4, 3), (5, 2), (6, 2)])
+@pytest.mark.parametrize("tp,cf,diss", [(P.CH, P.TWO_POINT_ROE, P.SIPG), (P.RA, P.TWO_POINT_LXF, P.BR2),
+                                        (P.RA, P.CENTRAL, P.SIPG), (P.IR, P.TWO_POINT_ROE, P.BR2)])
+@pytest.mark.parametrize("warp", [0, 1])
+def test_navier_stokes(p, n, tp, cf, diss, warp):
+    check(dict(SPLIT, **NS, dim=3, poly_degree=p, n_cells_1d=n, two_point_flux=tp, conv_flux=cf, diss_flux=diss,
+               grid_warp=warp), 7 * p + n)
+
+
+@pytest.mark.parametrize("dim,p,n", [(2, 1, 7), (2, 2, 3), (2, 4, 5), (2, 6, 3), (3, 1, 5), (3, 2, 4), (3, 3, 3),
+                                     (3, 4, 3), (3, 5, 2), (3, 6, 2)])
+@pytest.mark.parametrize("tp,cf", [(P.CH, P.TWO_POINT_ROE), (P.RA, P.ROE), (P.KG, P.TWO_POINT_LXF)])
+def test_curved_euler(dim, p, n, tp, cf):
+    lo, hi = (-1.0, 1.0) if dim == 2 else (0.0, 2 * np.pi)
+    check(dict(SPLIT, dim=dim, poly_degree=p, n_cells_1d=n, two_point_flux=tp, conv_flux=cf, grid_warp=1,
+               domain_left=lo, domain_right=hi), 11 * p + n)
+
+
 @pytest.mark.parametrize("dim,p,n", [(2, 1, 9), (2, 3, 5), (2, 6, 3), (3, 1, 5), (3, 3, 3), (3, 4, 3), (3, 6, 2)])
 @pytest.mark.parametrize("tp,cf", [(P.CH, P.TWO_POINT_ROE), (P.RA, P.LXF), (P.IR, P.TWO_POINT)])
 @pytest.mark.parametrize("bc", [1002, 1003, 1004, 1006, 1007])
