@@ -1564,38 +1564,38 @@ int dgx_batch_allocate(dgx_batch *b, int method, const double *dt)
         if (rc) return rc;
         for (int i : g.inst) b->variant[i] = g.tile + 1;
     }
-    // capture one RK step of every instance; within a stage the groups' launches are branches of
-    // the graph (forked from and joined into the batch stream), so the GPU can run blocks of
-    // several groups at once
+    // capture one RK step of every instance; each group's stages are a chain of their own (forked
+    // from and joined into the batch stream once a step, the groups share no data), so the GPU runs
+    // blocks of several groups at once and no group waits for another's stage
     const int ng = (int)b->groups.size();
     while ((int)b->side.size() < ng - 1) {
         hipStream_t st = nullptr;
         BHIPCHK(hipStreamCreate(&st));
         b->side.push_back(st);
     }
-    for (int k = 0; k < B.s * ng; ++k) {
+    for (int k = 0; k < ng; ++k) {
         hipEvent_t e = nullptr;
         BHIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         b->events.push_back(e);
     }
     BHIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     int rc = DGX_OK;
+    hipEvent_t *ev = b->events.data();  // [0]: fork, [k]: join of group k
+    if (ng > 1 && hipEventRecord(ev[0], b->stream) != hipSuccess) rc = DGX_ERR_HIP;
+    for (int k = 0; k < ng && rc == DGX_OK; ++k) {
+        BatchGroup &g = b->groups[k];
+        hipStream_t gs = k ? b->side[k - 1] : b->stream;
+        if (k && hipStreamWaitEvent(gs, ev[0], 0) != hipSuccess) rc = DGX_ERR_HIP;
+        const Ops1D &ops = b->inst[g.inst[0]]->ops;
+        for (int st = 0; st < B.s && rc == DGX_OK; ++st)
+            rc = launch_line_batch(g.dim, g.n, g.precision, g.generic, g.tile, g.blocks, g.nblocks, g.args[st], g.pcs, ops,
+                                   gs, nullptr);
+        if (!rc && k && hipEventRecord(ev[k], gs) != hipSuccess) rc = DGX_ERR_HIP;
+    }
+    for (int k = 1; k < ng && rc == DGX_OK; ++k)
+        if (hipStreamWaitEvent(b->stream, ev[k], 0) != hipSuccess) rc = DGX_ERR_HIP;
+    if (rc && b->err.empty()) b->err = "capture of the batched step failed";
     for (int st = 0; st < B.s && rc == DGX_OK; ++st) {
-        hipEvent_t *ev = b->events.data() + st * ng;  // [0]: fork, [k]: join of group k
-        if (ng > 1 && hipEventRecord(ev[0], b->stream) != hipSuccess) rc = DGX_ERR_HIP;
-        for (int k = 0; k < ng && rc == DGX_OK; ++k) {
-            BatchGroup &g = b->groups[k];
-            hipStream_t gs = k ? b->side[k - 1] : b->stream;
-            if (k && hipStreamWaitEvent(gs, ev[0], 0) != hipSuccess) rc = DGX_ERR_HIP;
-            const Ops1D &ops = b->inst[g.inst[0]]->ops;
-            if (!rc)
-                rc = launch_line_batch(g.dim, g.n, g.precision, g.generic, g.tile, g.blocks, g.nblocks, g.args[st], g.pcs, ops,
-                                       gs, nullptr);
-            if (!rc && k && hipEventRecord(ev[k], gs) != hipSuccess) rc = DGX_ERR_HIP;
-        }
-        for (int k = 1; k < ng && rc == DGX_OK; ++k)
-            if (hipStreamWaitEvent(b->stream, ev[k], 0) != hipSuccess) rc = DGX_ERR_HIP;
-        if (rc && b->err.empty()) b->err = "capture of the batched step failed";
         for (int i = 0; i < n && rc == DGX_OK; ++i) {
             dgx_ctx *c = b->inst[i];
             if (b->variant[i]) continue;
@@ -1689,6 +1689,11 @@ struct dgx_server {
     int max_active = 0, method = -1;
     Butcher B{};
     hipStream_t stream = nullptr;
+    // The groups of a step are independent through all its stages: they are spread over `stream` and
+    // these, so that groups of few blocks share the GPU (4 hardware queues in all).
+    static constexpr int SIDE = 3;
+    hipStream_t side[SIDE] = {nullptr, nullptr, nullptr};
+    hipEvent_t tables_ready = nullptr;
     int64_t next_id = 1;
     std::vector<Request> queue;     // FIFO
     std::vector<Request> active;
@@ -1849,15 +1854,41 @@ static int server_advance(dgx_server *s)
         }
     }
     if (bytes) SHIPCHK(hipMemcpyAsync(s->stage_dev, s->stage_host, bytes, hipMemcpyHostToDevice, s->stream));
+    // largest group first onto the stream with the fewest blocks so far
+    constexpr int NSTR = 1 + dgx_server::SIDE;
+    std::sort(groups.begin(), groups.end(), [](const G &a, const G &b) { return a.nblocks > b.nblocks; });
+    std::vector<int> on(groups.size());
+    int64_t load[NSTR] = {};
+    for (size_t k = 0; k < groups.size(); ++k) {
+        on[k] = (int)(std::min_element(load, load + NSTR) - load);
+        load[on[k]] += groups[k].nblocks;
+    }
+    SHIPCHK(hipEventRecord(s->tables_ready, s->stream));  // tables, and what admission enqueued
+    for (int k = 1; k < NSTR; ++k)
+        if (load[k]) SHIPCHK(hipStreamWaitEvent(s->side[k - 1], s->tables_ready, 0));
+    // waits for every stream that got work, also where a launch failed: the staging buffer and the
+    // requests' buffers are used again after this
+    auto settle = [&]() {
+        hipError_t e = hipStreamSynchronize(s->stream);
+        for (int k = 1; k < NSTR; ++k)
+            if (load[k]) {
+                const hipError_t e2 = hipStreamSynchronize(s->side[k - 1]);
+                if (e == hipSuccess) e = e2;
+            }
+        return e;
+    };
     for (int st = 0; st < S; ++st) {
-        for (G &g : groups) {
+        for (size_t gi = 0; gi < groups.size(); ++gi) {
+            G &g = groups[gi];
             const int m = (int)g.members.size();
             const Ops1D &ops = s->active[g.members[0]].c->ops;
+            const hipStream_t gs = on[gi] ? s->side[on[gi] - 1] : s->stream;
             int rc = launch_line_batch(g.dim, g.n, g.precision, g.generic, g.tile, (const BatchBlock *)(s->stage_dev + g.off_blocks),
                                        g.nblocks, (const StageArgs *)(s->stage_dev + g.off_args) + st * m,
-                                       (const PhysConst *)(s->stage_dev + g.off_pcs), ops, s->stream, nullptr);
+                                       (const PhysConst *)(s->stage_dev + g.off_pcs), ops, gs, nullptr);
             if (rc) {
                 s->err = "batched stage launch failed";
+                (void)settle();
                 return rc;
             }
         }
@@ -1869,11 +1900,12 @@ static int server_advance(dgx_server *s)
             if (!rc) rc = launch_stage(c, args[k][st]);
             if (rc) {
                 s->err = c->err;
+                (void)settle();
                 return rc;
             }
         }
     }
-    SHIPCHK(hipStreamSynchronize(s->stream));  // also releases the staging buffer
+    SHIPCHK(settle());  // also releases the staging buffer
     for (int k = 0; k < na; ++k) {
         Request &q = s->active[k];
         ++q.c->iteration;
@@ -1929,6 +1961,14 @@ int64_t dgx_request_bytes(const dgx_request *r, int method)
     return b;
 }
 
+static void server_free_streams(dgx_server *s)
+{
+    if (s->tables_ready) (void)hipEventDestroy(s->tables_ready);
+    for (hipStream_t st : s->side)
+        if (st) (void)hipStreamDestroy(st);
+    if (s->stream) (void)hipStreamDestroy(s->stream);
+}
+
 int dgx_server_create(int64_t hbm_budget_bytes, int max_active, int method, dgx_server **out)
 {
     if (!out || hbm_budget_bytes <= 0 || max_active < 1) return DGX_ERR_INVALID;
@@ -1944,9 +1984,16 @@ int dgx_server_create(int64_t hbm_budget_bytes, int max_active, int method, dgx_
         delete s;
         return DGX_ERR_HIP;
     }
+    bool ok = hipEventCreateWithFlags(&s->tables_ready, hipEventDisableTiming) == hipSuccess;
+    for (hipStream_t &st : s->side) ok = ok && hipStreamCreate(&st) == hipSuccess;
+    if (!ok) {
+        server_free_streams(s);
+        delete s;
+        return DGX_ERR_HIP;
+    }
     // the budget plus room for the per-request status words and 256-byte alignment of each buffer
     if (s->arena.init(hbm_budget_bytes + (16ll << 20) + 8192ll * max_active) != DGX_OK) {
-        (void)hipStreamDestroy(s->stream);
+        server_free_streams(s);
         delete s;
         return DGX_ERR_HIP;
     }
@@ -1962,7 +2009,7 @@ int dgx_server_destroy(dgx_server *s)
     s->arena.release();
     (void)hipHostFree(s->stage_host);
     (void)hipFree(s->stage_dev);
-    (void)hipStreamDestroy(s->stream);
+    server_free_streams(s);
     delete s;
     return DGX_OK;
 }
