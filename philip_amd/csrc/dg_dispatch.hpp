@@ -180,14 +180,18 @@ int launch_aux_dn(dgx_ctx *c, const double *u)
 {
     using S = Shape<D, N>;
     const int blocks = (c->ncells + S::EPB - 1) / S::EPB;
-    if (c->P.precision == DGX_MIXED)
-        hipLaunchKernelGGL((aux_kernel<D, N, float>), dim3(blocks), dim3(S::BLOCK), 0, c->stream, u, c->auxf_dev[0],
-                           c->auxf_dev[1], c->auxf_dev[2], c->nbr_dev, c->ncells, 1.0 / c->h, c->ops, c->pc,
+    auto go = [&](auto cc, auto *q0, auto *q1, auto *q2) {
+        using Q = std::remove_pointer_t<decltype(q0)>;
+        hipLaunchKernelGGL((aux_kernel<D, N, Q, decltype(cc)::value>), dim3(blocks), dim3(S::BLOCK), 0, c->stream, u,
+                           q0, q1, q2, c->nbr_dev, c->ncells, 1.0 / c->h, c->ops, c->pc,
                            c->curv ? c->met_dev : nullptr);
-    else
-        hipLaunchKernelGGL((aux_kernel<D, N, double>), dim3(blocks), dim3(S::BLOCK), 0, c->stream, u, c->aux_dev[0],
-                           c->aux_dev[1], c->aux_dev[2], c->nbr_dev, c->ncells, 1.0 / c->h, c->ops, c->pc,
-                           c->curv ? c->met_dev : nullptr);
+    };
+    auto grid = [&](auto *q0, auto *q1, auto *q2) {
+        if (c->curv) go(std::true_type{}, q0, q1, q2);
+        else go(std::false_type{}, q0, q1, q2);
+    };
+    if (c->P.precision == DGX_MIXED) grid(c->auxf_dev[0], c->auxf_dev[1], c->auxf_dev[2]);
+    else grid(c->aux_dev[0], c->aux_dev[1], c->aux_dev[2]);
     return check_launch(c, "aux_kernel");
 }
 

@@ -129,7 +129,7 @@ __device__ __forceinline__ int node_with(int i, int k, int l)
 // Streaming access to the RK registers: each value is read or written once per
 // stage and the registers together exceed the caches, so the stage kernels
 // mark these accesses non-temporal (STREAM_NT) to keep L2 for the neighbour
-// face traces.
+// face traces, but for the store of the next stage's state (stage_epilogue).
 constexpr bool STREAM_NT = true;
 __device__ __forceinline__ double ld_stream(const double *p)
 {
@@ -184,16 +184,20 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &
             n1 += a.beta * r;
             st_stream(a.s2 + idx, s2);
             if (a.lsrk_first) st_stream(a.s3 + idx, s1);
-            st_stream(a.s1_out + idx, n1);
+            // the next stage's state: on the box it is stored to stay in the last-level cache for that
+            // stage's read (TGV p=3 32^3 stage, FP64 117 -> 108 us, mixed 98 -> 91.5 us; S2 as well: no
+            // further gain); on a curvilinear grid the metric terms need the cache more (146 us, 154 us
+            // with this store)
+            if (a.met) st_stream(a.s1_out + idx, n1);
+            else a.s1_out[idx] = n1;
             if (a.s4) a.s4[idx] = (a.lsrk_first ? s1 : a.s4[idx]) + a.bhat * r;
         }
     } else {
-        const bool pf_b = std::is_same<T, double>::value && use_pf;
         for (int s = 0; s < NS; ++s) {
             const long idx = base + s * NP;
             const double kk = dudt[s];
-            // FP64 line kernels: the accumulator and u_n already loaded by the caller into pf2 / pf3
-            double accv = pf_b ? pf2[s] : (a.first_stage ? (a.acc_zero ? 0.0 : a.u0[idx]) : a.acc[idx]);
+            // use_pf: the accumulator and u_n already loaded by the caller into pf2 / pf3
+            double accv = use_pf ? pf2[s] : (a.first_stage ? (a.acc_zero ? 0.0 : a.u0[idx]) : a.acc[idx]);
             accv += a.b_dt * kk;
             a.acc_out[idx] = accv;
             if (a.k_store) a.k_store[idx] = kk;
@@ -207,7 +211,7 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &
                 }
                 if (a_cur != 0.0) st += a_cur * kk;
                 st *= a.dt;
-                st += 1.0 * (pf_b ? pf3[s] : a.u0[idx]);
+                st += 1.0 * (use_pf ? pf3[s] : a.u0[idx]);
                 a.u_next[idx] = st;
             }
         }
@@ -218,10 +222,10 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &
 //   q_d = (1/h) [ D_d u + (1/w_0) (u_hat - u) n_d ]  on faces normal to d, u_hat = {{u}}.
 // Q: storage type of q (double for the FP64 path, float for the mixed path, whose
 // kernels evaluate the viscous fluxes in float).
-// met: curvilinear grid (the metric terms [cell][dim*dim + 1][node]; null on the affine box):
+// CV: curvilinear grid, met its metric terms [cell][dim*dim + 1][node] (null on the affine box):
 //   q_k = (1/J) [ sum_j C[k][j] D_j u + (1/w_0) (u_hat - u) N_k ] with N the face's physical normal
 //   C n_ref at the node of the face's owner (the lower cell index; this cell on a boundary).
-template <int D, int N, typename Q>
+template <int D, int N, typename Q, bool CV>
 __global__ void __launch_bounds__((Shape<D, N>::BLOCK))
 aux_kernel(const double *__restrict__ u, Q *__restrict__ q0, Q *__restrict__ q1,
            Q *__restrict__ q2, const int *__restrict__ nbr, int ncells, double inv_h, Ops1D ops, PhysConst pc,
@@ -232,25 +236,37 @@ aux_kernel(const double *__restrict__ u, Q *__restrict__ q0, Q *__restrict__ q1,
     __shared__ double sU[EPB][NS][NP];
     const int tid = threadIdx.x;
     const int le = tid / NP, i = tid % NP;
-    const int e = blockIdx.x * EPB + le;
+    const int e = xcd_block() * EPB + le;
     const bool active = (le < EPB) && (e < ncells);
-    double ui[NS];
+    int c[3] = {0, 0, 0};
+    node_coords<D, N>(i, c);
+    // the neighbours' states at this node's faces (at most one per direction) are loaded with the own
+    // state: fetched in the direction loop, index then state, they were six round trips to memory one
+    // after the other (Navier-Stokes p=5 16^3: 43 -> 30 us, curved 66 -> 36 us)
+    double ui[NS], un[D][NS];
+    int nb[D];
     if (active) {
-        for (int s = 0; s < NS; ++s) {
-            ui[s] = u[((long)e * NS + s) * NP + i];
-            sU[le][s][i] = ui[s];
+#pragma unroll
+        for (int d = 0; d < D; ++d) nb[d] = nbr[e * 2 * D + 2 * d + (c[d] == N - 1 ? 1 : 0)];
+        for (int s = 0; s < NS; ++s) ui[s] = u[((long)e * NS + s) * NP + i];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const bool face = (c[d] == 0 || c[d] == N - 1) && nb[d] >= 0;
+            const int j = node_with<D, N>(i, d, c[d] == 0 ? N - 1 : 0);
+            if (face)
+                for (int s = 0; s < NS; ++s) un[d][s] = u[((long)nb[d] * NS + s) * NP + j];
         }
+        for (int s = 0; s < NS; ++s) sU[le][s][i] = ui[s];
     }
     __syncthreads();
     if (!active) return;
-    int c[3];
-    node_coords<D, N>(i, c);
     Q *qout[3] = {q0, q1, q2};
     constexpr int MS = D * D + 1;
-    double qp[D][NS];  // curvilinear grid: J times the physical gradient
-    if (met)
+    double qp[CV ? D : 1][NS];  // curvilinear grid: J times the physical gradient
+    if constexpr (CV)
         for (int k = 0; k < D; ++k)
             for (int s = 0; s < NS; ++s) qp[k][s] = 0.0;
+#pragma unroll
     for (int d = 0; d < D; ++d) {
         double g[NS];
         for (int s = 0; s < NS; ++s) {
@@ -258,43 +274,40 @@ aux_kernel(const double *__restrict__ u, Q *__restrict__ q0, Q *__restrict__ q1,
             for (int l = 0; l < N; ++l) acc += ops.D[c[d]][l] * sU[le][s][node_with<D, N>(i, d, l)];
             g[s] = acc;
         }
-        if (met)
+        if constexpr (CV)
             for (int k = 0; k < D; ++k) {
                 const double ckd = met[((long)e * MS + k * D + d) * NP + i];
                 for (int s = 0; s < NS; ++s) qp[k][s] += ckd * g[s];
             }
-        for (int side = 0; side < 2; ++side) {
-            if (c[d] != (side ? N - 1 : 0)) continue;
-            const int nb = nbr[e * 2 * D + 2 * d + side];
+        if (c[d] == 0 || c[d] == N - 1) {
+            const int side = c[d] == N - 1 ? 1 : 0;
             const int j = node_with<D, N>(i, d, side ? 0 : N - 1);
             const double sgn = side ? 1.0 : -1.0;
             // a wall face (nb < 0: -type): the viscous wall state of the node
             // (assemble_boundary_term_auxiliary_equation, strong_dg.cpp:790-870)
-            double ub[NS];
-            if (nb < 0) visc_wall_state<double, D>(-nb, ui, pc, ub);
+            if (nb[d] < 0) visc_wall_state<double, D>(-nb[d], ui, pc, un[d]);
             double lift[NS];
             for (int s = 0; s < NS; ++s) {
-                const double un = (nb < 0) ? ub[s] : u[((long)nb * NS + s) * NP + j];
-                const double avg = 0.5 * (ui[s] + un);
+                const double avg = 0.5 * (ui[s] + un[d][s]);
                 lift[s] = ops.inv_wb * (avg - ui[s]);
             }
-            if (met) {
+            if constexpr (CV) {
                 // the face's physical normal is the owner's (the lower cell index, or this cell on a
                 // boundary): sgn C[:, d] at the owner's face node
-                const bool own = nb < 0 || e < nb;
+                const bool own = nb[d] < 0 || e < nb[d];
                 for (int k = 0; k < D; ++k) {
                     const double nk = sgn * (own ? met[((long)e * MS + k * D + d) * NP + i]
-                                                 : met[((long)(nb < 0 ? 0 : nb) * MS + k * D + d) * NP + j]);
+                                                 : met[((long)(nb[d] < 0 ? 0 : nb[d]) * MS + k * D + d) * NP + j]);
                     for (int s = 0; s < NS; ++s) qp[k][s] += lift[s] * nk;
                 }
             } else {
                 for (int s = 0; s < NS; ++s) g[s] += lift[s] * sgn;
             }
         }
-        if (!met)
+        if constexpr (!CV)
             for (int s = 0; s < NS; ++s) qout[d][((long)e * NS + s) * NP + i] = Q(g[s] * inv_h);
     }
-    if (met) {
+    if constexpr (CV) {
         const double inv_j = 1.0 / met[((long)e * MS + D * D) * NP + i];
         for (int k = 0; k < D; ++k)
             for (int s = 0; s < NS; ++s) qout[k][((long)e * NS + s) * NP + i] = Q(qp[k][s] * inv_j);
