@@ -1491,8 +1491,7 @@ int dgx_batch_tile(const dgx_batch *b, int i, int *elements_per_block, int *wave
     if (!v) return DGX_OK;
     const dgx_ctx *c = b->inst[i];
     const bool fast = c->P.precision == DGX_MIXED;
-    const BatchTile t = batch_tile(c->dim, fast, v - 1);
-    *waves_bound = t.waves;
+    *waves_bound = c->dim == 2 ? batch_tile<2, 3>(fast, v - 1).waves : batch_tile<3, 3>(fast, v - 1).waves;
     return launch_line_batch(c->dim, c->n, c->P.precision, batch_generic(c), v - 1, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
                              elements_per_block, threads_per_block);
 }
@@ -1817,6 +1816,19 @@ static int server_advance(dgx_server *s)
         }
         g->members.push_back(k);
         grouped[k] = true;
+    }
+    for (G &g : groups) {
+        // a group that does not fill the chip in the default tile takes the small meshes'
+        int blocks = 0;
+        for (int k : g.members) blocks += (s->active[k].c->ncells + g.epb - 1) / g.epb;
+        if (g.tile == 0 && blocks <= s->active[g.members[0]].c->n_cu) {
+            int epb = 0;
+            if (launch_line_batch(g.dim, g.n, g.precision, g.generic, batch_tile_small(g.dim), nullptr, 0, nullptr,
+                                  nullptr, Ops1D{}, nullptr, &epb) == DGX_OK) {
+                g.tile = batch_tile_small(g.dim);
+                g.epb = epb;
+            }
+        }
     }
     // pack the tables
     int64_t bytes = 0;

@@ -24,119 +24,124 @@ inline int check_launch(dgx_ctx *c, const char *what)
     return DGX_OK;
 }
 
-// Split-form Euler on the box: with boundary faces or without, in FP64 with a kernel of its own for
-// the Kennedy-Gruber and Ismail-Roe fluxes.
-template <int D, int N, typename T>
+// Euler on the box in the line kernel, with boundary faces or without.
+template <int D, int N, typename T, int FORM>
 void line_dn(dgx_ctx *c, const StageArgs &a)
 {
     using LG = LineGeoS<D, N, T>;
-    auto go = [&](auto bc, auto gc) {
-        constexpr bool BND = decltype(bc)::value, GEN = decltype(gc)::value;
+    auto go = [&](auto bc) {
+        constexpr bool BND = decltype(bc)::value;
         const dim3 grid((c->ncells + LG::EPB - 1) / LG::EPB), block(LG::BLOCK);
         if constexpr (line_waves<D, N, T>() > 0)
-            hipLaunchKernelGGL((line_kernel_wb<D, N, T, line_waves<D, N, T>(), BND, GEN>), grid, block, 0, c->stream,
+            hipLaunchKernelGGL((line_kernel_wb<D, N, T, line_waves<D, N, T>(), BND, FORM>), grid, block, 0, c->stream,
                                a, c->ops, c->pc);
         else
-            hipLaunchKernelGGL((line_kernel<D, N, T, BND, GEN>), grid, block, 0, c->stream, a, c->ops, c->pc);
+            hipLaunchKernelGGL((line_kernel<D, N, T, BND, FORM>), grid, block, 0, c->stream, a, c->ops, c->pc);
     };
-    auto pick = [&](auto gc) {
-        if (c->has_boundary) go(std::true_type{}, gc);
-        else go(std::false_type{}, gc);
-    };
-    if constexpr (std::is_same<T, double>::value) {
-        if (c->pc.two_point < 2) return pick(std::true_type{});
+    if (c->has_boundary) {
+        go(std::true_type{});
+        return;
     }
-    pick(std::false_type{});
-}
-
-template <int D, int N, typename T>
-void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
-{
-    const bool split = c->P.use_split_form != 0;
-    const bool nsv = c->P.pde == DGX_NAVIER_STOKES;
-    const bool bnd = c->has_boundary;
-    if constexpr (std::is_same<T, double>::value) {
-        // FP64 Chandrashekar / Ranocha split form with the viscous terms or on a curvilinear grid, no
-        // boundary faces
-        if (split && !bnd && (nsv || c->curv) && c->pc.two_point >= 2) {
-            auto go = [&](auto vc, auto cc) {
-                constexpr bool V = decltype(vc)::value, CV = decltype(cc)::value;
-                using LV = LineGeoK<D, N, T, V>;
-                hipLaunchKernelGGL((line64_kernel<D, N, V, CV>), dim3((c->ncells + LV::EPB - 1) / LV::EPB),
-                                   dim3(LV::BLOCK), 0, c->stream, a, c->ops, c->pc);
-            };
-            if constexpr (D == 3) {
-                if (nsv) {
-                    if (c->curv) go(std::true_type{}, std::true_type{});
-                    else go(std::true_type{}, std::false_type{});
-                    return;
-                }
-            }
-            go(std::false_type{}, std::true_type{});
+    // A mesh of at most a block per compute unit is bound by the length of one block's chain, not by
+    // throughput.  Right-hand side, default -> small, at 0.4 blocks per unit: FP64 2D p=2 7.6 -> 5.6
+    // us, p=4 9.6 -> 5.9, p=6 11.1 -> 7.9; 3D p=1 10.6 -> 6.0, p=3 10.0 -> 6.1, p=5 12.2 -> 8.2; mixed 3D
+    // p=3 10.3 -> 6.2.  At one block per unit they meet (3D p=2 10.0 and 10.1, p=4 11.7 and 12.0); with
+    // 1.5 the small blocks are slower.  FP64 p=6 would spill.
+    if constexpr (FORM != FORM_GEN && !(D == 3 && N == 7 && std::is_same<T, double>::value)) {
+        using LS = LineGeoSmall<D, N, T>;
+        const int blocks = (c->ncells + LG::EPB - 1) / LG::EPB;
+        if (blocks <= c->n_cu) {
+            hipLaunchKernelGGL((line_kernel_small<D, N, T, FORM>), dim3((c->ncells + LS::EPB - 1) / LS::EPB),
+                               dim3(LS::BLOCK), 0, c->stream, a, c->ops, c->pc);
             return;
         }
     }
-    if (c->curv) {  // curvilinear grid: stage2_kernel with the metric terms, boundaries included
-        if constexpr (D == 3) {
-            if (nsv) {
-                if (split)
-                    hipLaunchKernelGGL((stage2_kernel<D, N, true, true, T, true, true>), grid, block, 0, c->stream, a,
-                                       c->ops, c->pc);
-                else
-                    hipLaunchKernelGGL((stage2_kernel<D, N, false, true, T, true, true>), grid, block, 0, c->stream,
-                                       a, c->ops, c->pc);
-                return;
-            }
+    go(std::false_type{});
+}
+
+// Stage kernel of a context.  FP64: the line kernel, but for walls with the viscous terms, boundary
+// faces on a curvilinear grid, and Kennedy-Gruber or Ismail-Roe fluxes with the viscous terms or on a
+// curvilinear grid, which are stage2_kernel's.  Mixed: the line kernel for the periodic split form and
+// for Euler boundary faces on the box, stage2_kernel for the rest.
+template <int D, int N, typename T>
+void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
+{
+    constexpr bool FP64 = std::is_same<T, double>::value;
+    const bool split = c->P.use_split_form != 0, bnd = c->has_boundary, curv = c->curv;
+    const bool nsv = D == 3 && c->P.pde == DGX_NAVIER_STOKES;
+    if (!nsv && !curv) {
+        if constexpr (FP64) {
+            if (!split) return line_dn<D, N, T, FORM_CONS>(c, a);
+            if (c->pc.two_point < 2) return line_dn<D, N, T, FORM_GEN>(c, a);
         }
-        if (split)
-            hipLaunchKernelGGL((stage2_kernel<D, N, true, false, T, true, true>), grid, block, 0, c->stream, a, c->ops,
-                               c->pc);
-        else
-            hipLaunchKernelGGL((stage2_kernel<D, N, false, false, T, true, true>), grid, block, 0, c->stream, a,
-                               c->ops, c->pc);
+        if (split) return line_dn<D, N, T, FORM_EC>(c, a);
+    }
+    if constexpr (FP64) {
+        if ((nsv || curv) && !bnd && (!split || c->pc.two_point >= 2)) {
+            auto go = [&](auto vc, auto cc, auto fc) {
+                constexpr bool V = decltype(vc)::value, CV = decltype(cc)::value;
+                constexpr int FORM = decltype(fc)::value ? FORM_CONS : FORM_EC;
+                using LV = LineGeoK<D, N, T, V>;
+                hipLaunchKernelGGL((line64_kernel<D, N, V, CV, FORM>), dim3((c->ncells + LV::EPB - 1) / LV::EPB),
+                                   dim3(LV::BLOCK), 0, c->stream, a, c->ops, c->pc);
+            };
+            auto form = [&](auto vc, auto cc) {
+                if (split) go(vc, cc, std::false_type{});
+                else go(vc, cc, std::true_type{});
+            };
+            if constexpr (D == 3) {
+                if (nsv) {
+                    if (curv) form(std::true_type{}, std::true_type{});
+                    else form(std::true_type{}, std::false_type{});
+                    return;
+                }
+            }
+            return form(std::false_type{}, std::true_type{});
+        }
+    } else if constexpr (D == 3) {
+        if (nsv && split && !curv && !bnd) {
+            using LV = LineGeoK<D, N, T, true>;
+            const dim3 vgrid((c->ncells + LV::EPB - 1) / LV::EPB), vblock(LV::BLOCK);
+            if constexpr (N == 6)
+                hipLaunchKernelGGL((line_kernel_ns_w4<D, N>), vgrid, vblock, 0, c->stream, a, c->ops, c->pc);
+            else
+                hipLaunchKernelGGL((line_kernel_ns<D, N>), vgrid, vblock, 0, c->stream, a, c->ops, c->pc);
+            return;
+        }
+    }
+    auto go2 = [&](auto sc, auto vc, auto bc, auto cc) {
+        hipLaunchKernelGGL((stage2_kernel<D, N, decltype(sc)::value, decltype(vc)::value, T, decltype(bc)::value,
+                                          decltype(cc)::value>),
+                           grid, block, 0, c->stream, a, c->ops, c->pc);
+    };
+    const std::true_type yes{};
+    const std::false_type no{};
+    if constexpr (D == 3) {
+        if (nsv && curv) {
+            if (split) go2(yes, yes, yes, yes);
+            else go2(no, yes, yes, yes);
+            return;
+        }
+        if (nsv && bnd) {
+            if (split) go2(yes, yes, yes, no);
+            else go2(no, yes, yes, no);
+            return;
+        }
+        if (nsv) {
+            // FP64: Kennedy-Gruber or Ismail-Roe; mixed: the conservative form
+            if constexpr (FP64) go2(yes, yes, no, no);
+            else go2(no, yes, no, no);
+            return;
+        }
+    }
+    if (curv) {
+        if (split) go2(yes, no, yes, yes);
+        else go2(no, no, yes, yes);
         return;
     }
-    if constexpr (D == 3) {
-        if (nsv && bnd) {
-            // Navier-Stokes with walls: stage2_kernel at both precisions
-            if (split)
-                hipLaunchKernelGGL((stage2_kernel<D, N, true, true, T, true>), grid, block, 0, c->stream, a, c->ops,
-                                   c->pc);
-            else
-                hipLaunchKernelGGL((stage2_kernel<D, N, false, true, T, true>), grid, block, 0, c->stream, a,
-                                   c->ops, c->pc);
-        } else if (split && nsv) {
-            if constexpr (std::is_same<T, float>::value) {
-                using LV = LineGeoK<D, N, T, true>;
-                const dim3 vgrid((c->ncells + LV::EPB - 1) / LV::EPB), vblock(LV::BLOCK);
-                if constexpr (N == 6)
-                    hipLaunchKernelGGL((line_kernel_ns_w4<D, N>), vgrid, vblock, 0, c->stream, a, c->ops, c->pc);
-                else
-                    hipLaunchKernelGGL((line_kernel_ns<D, N>), vgrid, vblock, 0, c->stream, a, c->ops, c->pc);
-            } else {
-                hipLaunchKernelGGL((stage2_kernel<D, N, true, true, T>), grid, block, 0, c->stream, a, c->ops,
-                                   c->pc);
-            }
-        }
-        else if (!split && nsv)
-            hipLaunchKernelGGL((stage2_kernel<D, N, false, true, T>), grid, block, 0, c->stream, a, c->ops, c->pc);
-        else if (split) {
-            line_dn<D, N, T>(c, a);
-        } else if (bnd) {
-            hipLaunchKernelGGL((stage2_kernel<D, N, false, false, T, true>), grid, block, 0, c->stream, a, c->ops,
-                               c->pc);
-        } else {
-            hipLaunchKernelGGL((stage2_kernel<D, N, false, false, T>), grid, block, 0, c->stream, a, c->ops, c->pc);
-        }
-    } else {
-        if (split) {
-            line_dn<D, N, T>(c, a);
-        } else if (bnd) {
-            hipLaunchKernelGGL((stage2_kernel<D, N, false, false, T, true>), grid, block, 0, c->stream, a, c->ops,
-                               c->pc);
-        } else {
-            hipLaunchKernelGGL((stage2_kernel<D, N, false, false, T>), grid, block, 0, c->stream, a, c->ops, c->pc);
-        }
+    if constexpr (!FP64) {  // conservative Euler on the box
+        if (bnd) go2(no, no, yes, no);
+        else go2(no, no, no, no);
     }
 }
 
@@ -195,7 +200,7 @@ int launch_aux_dn(dgx_ctx *c, const double *u)
     return check_launch(c, "aux_kernel");
 }
 
-template <int D, int N, typename T, int ES, int W, bool XJ, bool GEN>
+template <int D, int N, typename T, int ES, int W, int XJ, bool GEN>
 int line_batch_es(const BatchBlock *blocks, int nblocks, const StageArgs *args, const PhysConst *pcs,
                   const Ops1D &ops, hipStream_t st, int *epb, int *threads)
 {
@@ -223,17 +228,17 @@ int line_batch_t(int tile, const BatchBlock *blocks, int nblocks, const StageArg
     constexpr bool F = std::is_same<T, float>::value;
 #define LBT_CASE(V)                                                                                              \
     case V:                                                                                                      \
-        return line_batch_es<D, N, T, batch_tile(D, F, V).es, batch_tile(D, F, V).waves, batch_tile(D, F, V).xj, GEN>( \
+        return line_batch_es<D, N, T, batch_tile<D, N>(F, V).es, batch_tile<D, N>(F, V).waves, batch_tile<D, N>(F, V).xj, GEN>( \
             blocks, nblocks, args, pcs, ops, st, epb, threads);
     if constexpr (D == 2) {
         switch (tile) {
             LBT_CASE(0) LBT_CASE(1) LBT_CASE(2) LBT_CASE(3) LBT_CASE(4) LBT_CASE(5)
-            LBT_CASE(6) LBT_CASE(7) LBT_CASE(8) LBT_CASE(9) LBT_CASE(10) LBT_CASE(11)
+            LBT_CASE(6) LBT_CASE(7) LBT_CASE(8) LBT_CASE(9) LBT_CASE(10) LBT_CASE(11) LBT_CASE(12)
         default: return DGX_ERR_UNSUPPORTED;
         }
     } else {
         switch (tile) {
-            LBT_CASE(0) LBT_CASE(1)
+            LBT_CASE(0) LBT_CASE(1) LBT_CASE(2)
         default: return DGX_ERR_UNSUPPORTED;
         }
     }

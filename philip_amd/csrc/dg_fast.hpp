@@ -369,6 +369,27 @@ __device__ __forceinline__ void roe_fast(const NodeC<T, D> &L, const NodeC<T, D>
     for (int s = 0; s < D + 2; ++s) out[s] = T(-0.5) * A[s];
 }
 
+// Convective flux of a cached node along e_K or (CV) contracted with nv.
+template <int D, int K, bool CV>
+__device__ __forceinline__ void convective_flux64(const NodeC<double, D> &q, const double *nv, double *f)
+{
+    double vn;
+    if constexpr (CV) {
+        vn = q.vel[0] * nv[0];
+        for (int k = 1; k < D; ++k) vn += q.vel[k] * nv[k];
+    } else {
+        vn = q.vel[K];
+    }
+    const double m = q.u[0] * vn;
+    f[0] = m;
+    for (int k = 0; k < D; ++k) {
+        f[1 + k] = m * q.vel[k];
+        if constexpr (CV) f[1 + k] += q.p * nv[k];
+        else if (k == K) f[1 + k] += q.p;
+    }
+    f[D + 1] = m * q.h;
+}
+
 // Roe-Pike dissipation with Harten's entropy fix in double, -1/2 of it added to out: along the unit
 // normal n (CV) or sgn e_K.  co0 + co3 and (co3 - co0) c are formed once and shared by every state.
 template <int D, int K, bool CV>
@@ -464,8 +485,19 @@ __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const Node
         if constexpr (!GEN) {
             ec_flux64<D, K, CV>(L, R, n, fc, out);
         } else {
-            if (first) other_flux64<D, K, CV>(L, R, n, pc, out);
-            else other_flux64<D, K, CV>(R, L, n, pc, out);
+            // ordered by value: a branch would run both orders in a wave that holds both
+            NodeC<double, D> a, b;
+            a.u[0] = first ? L.u[0] : R.u[0];
+            b.u[0] = first ? R.u[0] : L.u[0];
+            for (int k = 0; k < D; ++k) {
+                a.vel[k] = first ? L.vel[k] : R.vel[k];
+                b.vel[k] = first ? R.vel[k] : L.vel[k];
+            }
+            a.p = first ? L.p : R.p;
+            b.p = first ? R.p : L.p;
+            a.h = first ? L.h : R.h;
+            b.h = first ? R.h : L.h;
+            other_flux64<D, K, CV>(a, b, n, pc, out);
         }
         if constexpr (!CV)
             for (int s = 0; s < D + 2; ++s) out[s] *= sgn;

@@ -48,21 +48,25 @@ namespace dgx {
 constexpr bool LINE_PREFETCH_RK_F = true;
 constexpr bool LINE_PREFETCH_RK_D = false;
 template <int D, int N> constexpr bool line_late_prefetch_d() { return !(D == 3 && N == 6); }
-// ES: elements per block relative to the 256-node default (ES > 0: ES times,
-// ES < 0: 1/|ES|); per-element strides do not depend on it.  XJ: the block has a
-// thread for every item of the line phase (one item pass, the extra threads idle in
-// the node phases) instead of one thread per node.
-template <int D, int N, typename T, int ES = 1, bool V = false, bool XJ = false> struct LineGeo {
+// ES: elements per block relative to the 256-node default (0 < ES < 64: ES times, ES < 0: 1/|ES|), or
+// their number (ES = 64 + elements); per-element strides do not depend on it.  XJ: threads of the
+// block: LINE_NODES one per node; LINE_ITEMS one for every item of the line phase (one item pass, the
+// extra threads idle in the node phases); LINE_WAVES the same with the items of each direction, part
+// and kind starting at a wave of their own, so that no wave runs two of them one after the other
+// (small meshes: threads cost nothing there, the longest chain does).
+enum LineThreads { LINE_NODES = 0, LINE_ITEMS = 1, LINE_WAVES = 2 };
+template <int D, int N, typename T, int ES = 1, bool V = false, int XJ = LINE_NODES> struct LineGeo {
     using G = Geo<D, N>;
     static constexpr int NP = G::NP, NS = D + 2, NL = G::NL;
-    static constexpr int EPB = ES > 0 ? G::EPB * ES : (G::EPB / -ES > 0 ? G::EPB / -ES : 1);
+    static constexpr int EPB = ES >= 64 ? ES - 64 : ES > 0 ? G::EPB * ES : (G::EPB / -ES > 0 ? G::EPB / -ES : 1);
     static constexpr bool FAST = std::is_same<T, float>::value;
     // node cache fields: rho, E, vel[D], p, b, |v|^2, sqrt(rho), c, h; FP64: without E (rho h - p)
     // and |v|^2
     static constexpr int NQ = FAST ? D + 8 : D + 6;
     // element strides padded to 1 mod 32 words so the stride-N lines of
-    // neighbouring elements fall in different LDS banks
-    static constexpr int pad1(int x) { return x + (33 - x % 32) % 32; }
+    // neighbouring elements fall in different LDS banks; FP64 p=1 in 3D, where that padding is a fifth
+    // of the block, to an odd number (60 -> 50 KB, two -> three blocks per CU: rhs of 40^3 49 -> 39 us)
+    static constexpr int pad1(int x) { return (D == 3 && N == 2 && !FAST) ? (x | 1) : x + (33 - x % 32) % 32; }
     // 3D, N = 4: node cache in the skewed order of qpos (the 16 x-lines of an element would
     // otherwise read 4 words apart, 4 lanes per bank pair); its float element stride is 16 mod 32
     // words so the two elements a 32-lane access spans take complementary bank halves.  At p=3
@@ -95,8 +99,13 @@ template <int D, int N, typename T, int ES = 1, bool V = false, bool XJ = false>
     static constexpr int ITEMS = EPB * D * NL * LS;
     static constexpr int FITEMS = EPB * NFN;
     static constexpr int round64(int x) { return ((x + 63) / 64) * 64; }
-    static constexpr int BLOCK = XJ ? round64(EPB * NP > ITEMS + FITEMS ? EPB * NP : ITEMS + FITEMS)
-                                    : round64(EPB * NP);
+    // LINE_WAVES: threads of one (direction, part)'s line items and of one direction's face items
+    static constexpr int PG = round64(EPB * NL), FG = round64(2 * EPB * NL);
+    static constexpr int larger(int x, int y) { return x > y ? x : y; }
+    static constexpr int BLOCK = XJ == LINE_WAVES ? larger(round64(EPB * NP), D * (LS * PG + FG))
+                                 : XJ == LINE_ITEMS ? round64(larger(EPB * NP, ITEMS + FITEMS))
+                                    // p = 6 Navier-Stokes, mixed: 441 line items, one per thread
+                                    : round64(V && N == 7 && ITEMS > EPB * NP ? ITEMS : EPB * NP);
     // Navier-Stokes (V): own viscous flux in every direction [direction][state][node] and the
     // neighbours' viscous flux along the face direction at their face nodes
     // [state][face][face node]; FP64 leaves out the density component, which is zero
@@ -108,6 +117,11 @@ template <int D, int N, typename T, int ES = 1, bool V = false, bool XJ = false>
     // cache's place (and what follows it) once every item has run
     static constexpr int SBUF = EPB * ESN + ((ESQ + ESFV + ESNV > ESV) ? EPB * (ESQ + ESFV + ESNV) : EPB * ESV);
 };
+
+// Volume form of an FP64 line kernel: Chandrashekar / Ranocha split form, the split form with one of
+// the other two-point fluxes (a kernel of its own: the generic evaluation sets the register count of
+// a kernel that holds both -- p=3: 153 VGPRs, the curved kernel 246), the conservative form.
+enum LineForm { FORM_EC = 0, FORM_GEN = 1, FORM_CONS = 2 };
 
 // Elements-per-block variant of the single-solve line kernel: 1 for Euler; for
 // Navier-Stokes (V) the 256-node default block halved until its LDS fits 64 KB
@@ -125,7 +139,10 @@ template <int D, int N, typename T, bool V> constexpr int line_es()
     }
 }
 template <int D, int N, typename T, bool V> using LineGeoK = LineGeo<D, N, T, line_es<D, N, T, V>(), V>;
-template <int D, int N, bool V, bool CV> constexpr int line64_waves() { return 2; }
+// Waves per SIMD line64_kernel is held to: on curvilinear grids up to p=5 three (stage, held to two ->
+// three: p=4 24^3 207 -> 187 us, p=5 16^3 146 -> 132 us, Navier-Stokes p=5 16^3 272 -> 254 us, p=3 the
+// same); on the box it takes 164 VGPRs at p=5 by itself, and p=6 is slower with a bound.
+template <int D, int N, bool V, bool CV> constexpr int line64_waves() { return CV && N <= 6 ? 3 : 2; }
 
 // ---- node cache in LDS ----------------------------------------------------
 // Position of node i (x fastest) in its element's cache.  3D, N = 4: the skewed order
@@ -256,17 +273,20 @@ template <int N, int LS, int H> __device__ __forceinline__ constexpr bool pair_i
     return idx >= H * NPAIR / LS && idx < (H + 1) * NPAIR / LS;
 }
 
-// FP64: two-point fluxes of part H of a line with the two-point flux TP (2 Chandrashekar, 3 Ranocha,
-// 0 the generic evaluation; a constant, so that an item's code holds one of them and loads what it
-// needs).  CV: contracted with the pair's average cofactor column, cm the nodes' columns.
-template <int D, int N, int K, int LS, int H, bool CV, int TP>
-__device__ __forceinline__ void pairs64(const Ops1D &ops, const PhysConst &pc, const FastConst<double> &fc0,
+// FP64: two-point fluxes of part H of a line; GEN: Kennedy-Gruber or Ismail-Roe.  CV: contracted with
+// the pair's average cofactor column, cm the nodes' columns.  Chandrashekar and Ranocha in one body
+// that asks for the flux per pair, or as two bodies behind one branch (fc.two_point a constant in
+// each): then their common loads, every node of the line, are hoisted above the branch and held, and
+// the pairs overlap more.  Stage, one body -> two: p=3 32^3 113 -> 125 us, curved p=4 24^3 207 -> 327
+// us, Navier-Stokes p=5 16^3 161 -> 168 us; p=4 24^3 145 -> 142 us, p=5 20^3 183 -> 171 us, p=6 16^3
+// 247 -> 232 us, 2D p=4 196 -> 191 us, p=5 268 -> 253 us, p=6 315 -> 286 us.  So two from p=4 for Euler
+// on the box (line_block), one otherwise.
+template <int D, int N, int K, int LS, int H, bool CV, bool GEN>
+__device__ __forceinline__ void pairs64(const Ops1D &ops, const PhysConst &pc, const FastConst<double> &fc,
                                         const double *sq, const double (&cm)[CV ? N : 1][D], int line,
                                         double (&acc)[N][D + 2])
 {
     constexpr int NP = Geo<D, N>::NP, NS = D + 2;
-    FastConst<double> fc = fc0;
-    if (TP) fc.two_point = TP;
 #pragma unroll
     for (int p0 = 0; p0 < N; ++p0) {
 #pragma unroll
@@ -278,7 +298,7 @@ __device__ __forceinline__ void pairs64(const Ops1D &ops, const PhysConst &pc, c
             double nv[D], F[NS];
             if constexpr (CV)
                 for (int m = 0; m < D; ++m) nv[m] = 0.5 * (cm[p0][m] + cm[p1][m]);
-            if constexpr (TP > 0) {
+            if constexpr (!GEN) {
                 ec_flux64<D, K, CV>(A, B, nv, fc, F);
             } else {
                 const double *qa = sq + qpos<D, N>(line_node<D, N>(K, line, p0)) + (D + 3) * NP;
@@ -324,6 +344,29 @@ __device__ __forceinline__ void pairs_f(const Ops1D &ops, const PhysConst &pc, c
 }
 
 // ---- Navier-Stokes terms (either precision) --------------------------------
+
+// FP64, conservative form: node a gets -sum_b D[a][b] F_K(u_b) (CV: contracted with the node's
+// cofactor column), part H of LS of the columns b.
+template <int D, int N, int K, int LS, int H, bool CV>
+__device__ __forceinline__ void cons_line64(const Ops1D &ops, const double *sq, const double (&cm)[CV ? N : 1][D],
+                                            int line, double (&acc)[N][D + 2])
+{
+    constexpr int NP = Geo<D, N>::NP, NS = D + 2;
+#pragma unroll
+    for (int b = H * N / LS; b < (H + 1) * N / LS; ++b) {
+        const double *q = sq + qpos<D, N>(line_node<D, N>(K, line, b));
+        NodeC<double, D> B;
+        double f[NS];
+        nodef_load_pair<D>(q, NP, B);
+        B.h = q[(D + 3) * NP];
+        convective_flux64<D, K, CV>(B, cm[CV ? b : 0], f);
+#pragma unroll
+        for (int a2 = 0; a2 < N; ++a2) {
+            const double dab = ops.D[a2][b];
+            for (int s = 0; s < NS; ++s) acc[a2][s] -= dab * f[s];
+        }
+    }
+}
 
 // Viscous part of the volume term along one line: node a gets -sum_b D[a][b] F_v,K(u_b, q_b)
 // (the conservative D-divergence of strong_dg.cpp:1386-1433 for the dissipative flux); sfv
@@ -459,7 +502,7 @@ __device__ __forceinline__ void face_f(const Ops1D &ops, const PhysConst &pc, co
 // changes its bits.  CV: along the physical normal C n_ref of the face's owner (the lower cell
 // index), scaled by its length.  trv (V): the neighbour's viscous flux along e_K, or (CV)
 // contracted with the owner's cofactor column.
-template <int D, int N, int K, bool V, bool CV, bool BND, bool GEN>
+template <int D, int N, int K, bool V, bool CV, bool BND, int FORM>
 __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, const PhysConst &pc,
                                        const FastConst<double> &fc, const FaceIn<double> &in, int le, int side, int fn,
                                        int e, int nb, int nbl, double (&out)[D + 2], double (&out_nb)[D + 2])
@@ -493,12 +536,29 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         node_fill<double, D>(qn, fc);
     }
     double fs[NS];
-    num_flux64<D, K, CV, GEN>(qi, qn, sgn, nh, own, fc, pc, fs);
+    num_flux64<D, K, CV, FORM == FORM_GEN>(qi, qn, sgn, nh, own, fc, pc, fs);
     const double iwb = ops.inv_wb;
     const double w = CV ? iwb * area : iwb;
     for (int s = 0; s < NS; ++s) {
         out[s] = -(w * fs[s]);
         out_nb[s] = -out[s];
+    }
+    if constexpr (FORM == FORM_CONS) {
+        // the strong form's interior flux, each side's with its own cofactor column
+        double ca[D], cb[D], fi_[NS], fj_[NS];
+        if constexpr (CV) {
+            const double *pa = a.met + (long)e * MS * NP + fi, *pb = a.met + (long)nb * MS * NP + fj;
+            for (int m = 0; m < D; ++m) {
+                ca[m] = pa[(m * D + K) * NP];
+                cb[m] = nbl >= 0 ? pb[(m * D + K) * NP] : 0.0;
+            }
+        }
+        convective_flux64<D, K, CV>(qi, ca, fi_);
+        convective_flux64<D, K, CV>(qn, cb, fj_);
+        for (int s = 0; s < NS; ++s) {
+            out[s] += (iwb * sgn) * fi_[s];
+            out_nb[s] -= (iwb * sgn) * fj_[s];
+        }
     }
     if constexpr (V) {
         // average of the one-sided viscous fluxes (antisymmetric between the sides) and, one-sided,
@@ -564,12 +624,10 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
 // One block's work: elements blk0 .. blk0 + EPB - 1 of the solve described by a.
 // V: Navier-Stokes (split convective form plus the viscous volume and surface
 // terms, with the lifted gradient a.aux computed beforehand).
-// CV (FP64): curvilinear grid, metric terms a.met.  BND: Euler boundary faces.  GEN (FP64): the
-// two-point flux is Kennedy-Gruber or Ismail-Roe, else Chandrashekar or Ranocha: a kernel of its own,
-// since the generic evaluation sets the register count of a kernel that holds both (p=3: 153 VGPRs,
-// the curved kernel 246).
-template <int D, int N, typename T, int ES, bool V = false, bool XJ = false, bool BND = false, bool CV = false,
-          bool GEN = false>
+// CV (FP64): curvilinear grid, metric terms a.met.  BND: Euler boundary faces.  FORM: volume form
+// (FP64; the mixed path's kernels hold every two-point flux).
+template <int D, int N, typename T, int ES, bool V = false, int XJ = LINE_NODES, bool BND = false, bool CV = false,
+          int FORM = FORM_EC>
 __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops, const PhysConst &pc, const int blk0)
 {
     using LG = LineGeo<D, N, T, ES, V, XJ>;
@@ -757,52 +815,91 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
     }
     __syncthreads();
 
+    const int lane = tid & 63, wv = tid >> 6;
+    auto face_wanted = [&](int fle, int f) {
+        const int nb = sNb[fle][f];
+        return blk0 + fle < a.ncells && !(in_block(nb, blk0 + fle) && nb < blk0 + fle);
+    };
     // ---------------- faces evaluated in this block ----------------------
     // Face side (le, f) is evaluated here unless its neighbour is an element
     // of this block with a lower index (that element evaluates the shared face
     // once for both).  Each wave builds the same list in its own LDS row,
     // ordered by direction so that a wave's face items mostly share one.
-    const int lane = tid & 63, wv = tid >> 6;
     int nface = 0;
-    for (int c0 = 0; c0 < NFS; c0 += 64) {
+    for (int c0 = 0; XJ != LINE_WAVES && c0 < NFS; c0 += 64) {
         const int id = c0 + lane;  // id = (k * EPB + le) * 2 + side
-        bool want = false;
-        if (id < NFS) {
-            const int kk = id / (2 * EPB), r = id % (2 * EPB);
-            const int fle = r >> 1, f = 2 * kk + (r & 1);
-            if (blk0 + fle < a.ncells) {
-                const int nb = sNb[fle][f];
-                want = !(in_block(nb, blk0 + fle) && nb < blk0 + fle);
-            }
-        }
+        const bool want = id < NFS && face_wanted((id % (2 * EPB)) >> 1, 2 * (id / (2 * EPB)) + (id & 1));
         const unsigned long long m = __ballot(want);
         if (want) sList[wv][nface + __popcll(m & ((1ull << lane) - 1ull))] = (short)id;
         nface += __popcll(m);
     }
 
-    // ---------------- phase L: pair-line items, then face items ----------
+    // ---------------- phase L: face items, then pair-line items ----------
+    // Faces first, so that no line sum is live while a face is evaluated (the line sums are held to
+    // the end of the phase): FP64 p=3 153 -> 121 VGPRs, three -> four waves per SIMD, stage 128 ->
+    // 112 us at 32^3; mixed p=4 24^3 122 -> 112 us, mixed Navier-Stokes p=5 16^3 stage 113 -> 107 us.
+    // The face
+    // items go to the threads from the first on, the line items from the last on, so the threads that
+    // have one item more are different ones.
+    // Mixed 3D Euler at p=3 and p=6: lines first and both kinds in one run of items, where the kernels'
+    // registers allow no further wave: rhs faces first -> this, p=3 32^3 72 -> 69 us, p=6 16^3 162 ->
+    // 126 us (lines and faces as two passes: 170 us).
+    constexpr bool FACES_FIRST = !(FAST && D == 3 && (N == 4 || N == 7) && !V) || XJ == LINE_WAVES;
     constexpr int PITEMS = LG::ITEMS;                          // (direction, part, element, line)
-    constexpr int JP = (PITEMS + BLOCK - 1) / BLOCK;           // slots that can hold a line item
-    constexpr int JT = (PITEMS + NFS * NL + BLOCK - 1) / BLOCK;
-    // V with in-block neighbours: the neighbour's side of a shared face is not the negated own
-    // side (the interior viscous flux is one-sided), so it is held separately
-    constexpr bool NBT = V && EPB > 1;
-    const int items = PITEMS + nface * NL;
+    constexpr int JP = (PITEMS + BLOCK - 1) / BLOCK;           // line items per thread
+    constexpr int JF = (NFS * NL + BLOCK - 1) / BLOCK;         // face items per thread
+    // this thread's line item j: direction and part kh = k * LS + h, element and line r
+    auto line_item = [&](int j, int &kh, int &r) {
+        if constexpr (XJ == LINE_WAVES) {
+            kh = tid / LG::PG;
+            r = tid % LG::PG;
+            return kh < D * LS && r < EPB * NL;
+        } else {
+            const int t = (FACES_FIRST ? BLOCK - 1 - tid : tid) + j * BLOCK;
+            kh = t / (EPB * NL);
+            r = t % (EPB * NL);
+            return t < PITEMS;
+        }
+    };
+    // this thread's face item j: direction and side of an element, face node
+    auto face_item = [&](int j, int &k, int &fle, int &side, int &fn) {
+        if constexpr (XJ == LINE_WAVES) {
+            const int u = tid - D * LS * LG::PG, r = u % LG::FG;
+            k = u / LG::FG;
+            fle = r / (2 * NL);
+            side = (r / NL) & 1;
+            fn = r % NL;
+            return u >= 0 && k < D && r < 2 * EPB * NL && face_wanted(fle, 2 * k + side);
+        } else {
+            const int t = tid + j * BLOCK - (FACES_FIRST ? 0 : PITEMS);
+            if (t < 0 || t >= nface * NL) return false;
+            const int id = sList[wv][t / NL], r = id % (2 * EPB);
+            k = id / (2 * EPB);
+            fle = r >> 1;
+            side = r & 1;
+            fn = t % NL;
+            return true;
+        }
+    };
+    // V or the conservative form with in-block neighbours: the neighbour's side of a shared face is
+    // not the negated own side (the strong form's interior flux is one-sided), so it is held
+    // separately
+    constexpr bool NBT = (V || FORM == FORM_CONS) && EPB > 1;
     const T pen = T(a.penalty);
-    T rp[JP][N][NS];
-#pragma unroll
-    for (int j = 0; j < JT; ++j) {
-        const int t = tid + j * BLOCK;
-        if (j < JP && t < PITEMS) {
+    auto line_pass = [&](int j, T(&rpj)[N][NS]) __attribute__((always_inline)) {
+        int kh, r;
+        if (line_item(j, kh, r)) {
             // t = ((k * LS + h) * EPB + element) * NL + line: direction k, part h of the line
-            const int kh = t / (EPB * NL), r = t % (EPB * NL);
             const int k = kh / LS, h = kh % LS;
             const int lle = r / NL, line = r % NL;
-            if (blk0 + lle >= a.ncells) continue;
+            if (blk0 + lle >= a.ncells) return;
             const T *q = sQ + lle * LG::ESQ;
-            auto pitem = [&](auto kc, auto hc) {
+            auto pitem = [&](auto kc, auto hc) __attribute__((always_inline)) {
                 constexpr int K = decltype(kc)::value, H = decltype(hc)::value;
-                T(&acc)[N][NS] = rp[j < JP ? j : 0];
+                T(&acc)[N][NS] = rpj;
+                // marks that differ per part keep the parts' code apart: merged, they read the operator
+                // tables through a pointer chosen per lane, from a copy of the tables in scratch
+                if constexpr (LS > 1) asm volatile("; part %0" ::"i"(3 * K + H));
                 if constexpr (FAST) {
                     pairs_f<T, D, N, K, LS, H>(ops, pc, fc, q, line, acc);
                     if constexpr (V) visc_line<D, N, K, T, LS, H>(ops, sFv + lle * LG::ESFV, line, acc);
@@ -818,16 +915,29 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
 #pragma unroll
                     for (int p = 0; p < N; ++p)
                         for (int s = 0; s < NS; ++s) acc[p][s] = 0.0;
-                    if constexpr (GEN) {
-                        pairs64<D, N, K, LS, H, CV, 0>(ops, pc, fc, q, cm, line, acc);
+                    if constexpr (FORM == FORM_CONS) {
+                        cons_line64<D, N, K, LS, H, CV>(ops, q, cm, line, acc);
+                    } else if constexpr (FORM == FORM_GEN) {
+                        pairs64<D, N, K, LS, H, CV, true>(ops, pc, fc, q, cm, line, acc);
                     } else {
-                        if (fc.two_point == 2) pairs64<D, N, K, LS, H, CV, 2>(ops, pc, fc, q, cm, line, acc);
-                        else pairs64<D, N, K, LS, H, CV, 3>(ops, pc, fc, q, cm, line, acc);
+                        if constexpr (!V && !CV && N >= 5) {
+                            FastConst<double> fk = fc;
+                            if (fc.two_point == 2) {
+                                fk.two_point = 2;
+                                pairs64<D, N, K, LS, H, CV, false>(ops, pc, fk, q, cm, line, acc);
+                            } else {
+                                fk.two_point = 3;
+                                pairs64<D, N, K, LS, H, CV, false>(ops, pc, fk, q, cm, line, acc);
+                            }
+                        } else {
+                            pairs64<D, N, K, LS, H, CV, false>(ops, pc, fc, q, cm, line, acc);
+                        }
                     }
                     if constexpr (V) visc_line64<D, N, K, LS, H, CV>(ops, sFv + lle * LG::ESFV, cm, line, acc);
                 }
+                if constexpr (LS > 1) asm volatile("; end of part %0" ::"i"(3 * K + H));
             };
-            auto pdir = [&](auto kc) {
+            auto pdir = [&](auto kc) __attribute__((always_inline)) {
                 if (h == 0) pitem(kc, std::integral_constant<int, 0>{});
                 else if (LS > 1 && h == 1) pitem(kc, std::integral_constant<int, (LS > 1 ? 1 : 0)>{});
                 else if (LS > 2) pitem(kc, std::integral_constant<int, (LS > 2 ? 2 : 0)>{});
@@ -835,23 +945,25 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
             if (k == 0) pdir(std::integral_constant<int, 0>{});
             else if (k == 1) pdir(std::integral_constant<int, 1>{});
             else if (D == 3) pdir(std::integral_constant<int, (D == 3 ? 2 : 1)>{});
-        } else if (t >= PITEMS && t < items) {
-            const int u = (t - PITEMS) / NL, fn = (t - PITEMS) % NL;
-            const int id = sList[wv][u];
-            const int k = id / (2 * EPB), r = id % (2 * EPB);
-            const int fle = r >> 1, side = r & 1;
+        }
+    };
+    T rp[JP][N][NS];
+    static_assert(JP <= 2, "line items per thread");
+    auto face_pass = [&](int j) __attribute__((always_inline)) {
+        int k, fle, side, fn;
+        if (face_item(j, k, fle, side, fn)) {
             const int nb = sNb[fle][2 * k + side];
             const int nbl = in_block(nb, blk0 + fle) ? nb - blk0 : -1;
             const int fo = (2 * k + side) * NL + fn;
             T *const slot = sN + fle * LG::ESN + fo;
             const FaceIn<T> in{sQ, sFv, slot, sNv + fle * LG::ESNV + fo, LG::NFN};
             T rf[NS], rfn[NS];
-            auto fitem = [&](auto kc) {
+            auto fitem = [&](auto kc) __attribute__((always_inline)) {
                 constexpr int K = decltype(kc)::value;
                 if constexpr (FAST)
                     face_f<T, D, N, K, V, BND>(ops, pc, fc, in, fle, side, fn, blk0 + fle, nb, nbl, pen, rf, rfn);
                 else
-                    face64<D, N, K, V, CV, BND, GEN>(a, ops, pc, fc, in, fle, side, fn, blk0 + fle, nb, nbl, rf, rfn);
+                    face64<D, N, K, V, CV, BND, FORM>(a, ops, pc, fc, in, fle, side, fn, blk0 + fle, nb, nbl, rf, rfn);
             };
             if (k == 0) fitem(std::integral_constant<int, 0>{});
             else if (k == 1) fitem(std::integral_constant<int, 1>{});
@@ -864,16 +976,32 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
                 for (int s = 0; s < NS; ++s) w2[s * LG::NFN] = NBT ? rfn[s] : -rf[s];
             }
         }
+    };
+    if constexpr (FACES_FIRST) {
+#pragma unroll
+        for (int j = 0; j < JF; ++j) face_pass(j);
+        line_pass(0, rp[0]);
+        if constexpr (JP > 1) line_pass(JP - 1, rp[JP - 1]);
+    } else {
+        static_assert(JP == 1, "lines first: one line item per thread");
+#pragma unroll
+        for (int j = 0; j < (PITEMS + NFS * NL + BLOCK - 1) / BLOCK; ++j) {
+            if (j == 0 && tid < PITEMS) line_pass(0, rp[0]);
+            else face_pass(j);
+        }
     }
     __syncthreads();  // node cache and traces consumed; their storage now takes the partials
-    constexpr bool LATE_PF = !PREFETCH && !FAST && line_late_prefetch_d<D, N>();
+    // FP64: the registers of the epilogue are read from here on; mixed: those of a Butcher stage (S2
+    // and S3 were loaded in phase A; not at p=6 in 3D, which spills; 2D p=3 512^2 RK4 stage 157 -> 128 us, Navier-Stokes p=5 16^3 147 ->
+    // 129 us with the lifted gradient)
+    constexpr bool LATE_PF = FAST ? (V || D == 2 || N != 7) : line_late_prefetch_d<D, N>();
     const bool late_pf = LATE_PF && active &&
-                         ((a.mode == MODE_LSRK && !a.lsrk_first) || a.mode == MODE_BUTCHER);
+                         ((!FAST && a.mode == MODE_LSRK && !a.lsrk_first) || a.mode == MODE_BUTCHER);
     // FP64 at N >= 4: the stage state is read again here for the epilogue (an L2 hit: the block
     // read it in phase A) instead of being held in registers through the line phase (TGV 32^3
     // p=3: 177 -> 170 us per stage, 64 -> 16 B/lane of spills; p=4 24^3 294 -> 244 us; at p=2
     // slower)
-    constexpr bool REREAD = LATE_PF && N >= 4;
+    constexpr bool REREAD = !FAST && LATE_PF && N >= 4;
     double ue[NS];
     if (REREAD && active && a.mode == MODE_LSRK)
         for (int s = 0; s < NS; ++s) ue[s] = a.u[((long)e * NS + s) * NP + i];
@@ -894,14 +1022,12 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
     // Line partials of one direction at a time into one [part][state][node] buffer: direction 0
     // stores, each later direction adds after a barrier, so every part's sum is ((d0 + d1) + d2)
     // in this order in every block layout.
-    auto line_out = [&](auto kc, bool add) {
+    auto line_out = [&](auto kc, bool add) __attribute__((always_inline)) {
         constexpr int KD = decltype(kc)::value;
 #pragma unroll
         for (int j = 0; j < JP; ++j) {
-            const int t = tid + j * BLOCK;
-            if (t >= PITEMS) continue;
-            const int kh = t / (EPB * NL), r = t % (EPB * NL);
-            if (kh / LS != KD) continue;
+            int kh, r;
+            if (!line_item(j, kh, r) || kh / LS != KD) continue;
             const int lle = r / NL, line = r % NL;
             if (blk0 + lle >= a.ncells) continue;
             T *v = sV + lle * LG::ESV + (kh % LS) * NS * NP;
@@ -956,31 +1082,48 @@ template <int D, int N, typename T> constexpr int line_es_single()
 }
 template <int D, int N, typename T> using LineGeoS = LineGeo<D, N, T, line_es_single<D, N, T>()>;
 
+// Small meshes: fewer elements per block, so that a mesh that cannot fill the chip spreads over more
+// of it, and LINE_WAVES threads, so that a thread's chain is one item long instead of two or three.
+// Elements per block: what fills half a wave per (direction, part) of line items.
+template <int D, int N> constexpr int line_es_small()
+{
+    return 64 + (D == 2 ? (N == 2 ? 16 : N == 3 ? 10 : N == 4 ? 8 : N == 5 ? 6 : N == 6 ? 5 : 4)
+                        : (N == 2 ? 8 : N == 3 ? 3 : N == 4 ? 2 : 1));
+}
+template <int D, int N, typename T> using LineGeoSmall = LineGeo<D, N, T, line_es_small<D, N>(), false, LINE_WAVES>;
+template <int D, int N, typename T, int FORM>
+__global__ void __launch_bounds__((LineGeoSmall<D, N, T>::BLOCK))
+line_kernel_small(StageArgs a, Ops1D ops, PhysConst pc)
+{
+    line_block<D, N, T, line_es_small<D, N>(), false, LINE_WAVES, false, false, FORM>(
+        a, ops, pc, xcd_block() * LineGeoSmall<D, N, T>::EPB);
+}
+
 // One solve: blocks in XCD-aware order over the element groups.  BND: the mesh has boundary
 // faces (a separate instantiation, so the periodic kernels carry no boundary code).
-template <int D, int N, typename T, bool BND = false, bool GEN = false>
+template <int D, int N, typename T, bool BND = false, int FORM = FORM_EC>
 __global__ void __launch_bounds__((LineGeoS<D, N, T>::BLOCK))
 line_kernel(StageArgs a, Ops1D ops, PhysConst pc)
 {
-    line_block<D, N, T, line_es_single<D, N, T>(), false, false, BND, false, GEN>(
+    line_block<D, N, T, line_es_single<D, N, T>(), false, LINE_NODES, BND, false, FORM>(
         a, ops, pc, xcd_block() * LineGeoS<D, N, T>::EPB);
 }
 // Waves per SIMD the single-solve 3D line kernel is held to (amdgpu_waves_per_eu; 0: the
-// compiler's choice).  The mixed path keeps the compiler's choice (a 4-wave bound at p=6 was
-// faster with an earlier, larger LDS layout; it now measures 296 against 278 us per stage at 16^3).
-// FP64 path at p=3..5: 3 (168 VGPRs; p=3 takes 153 and spills nothing, TGV p=3 32^3 140 us per
-// stage); at p=2 no change and at p=6 much slower (448 -> 724 us with an earlier form of the
-// fluxes), so those keep the compiler's choice.
+// compiler's choice).  The mixed path at p=3: 4, which it misses by one register otherwise (129).
+// FP64 path: 4 at p=3 (121 VGPRs, TGV 32^3 112 us per stage), 3 at p=4 and p=5 (156 VGPRs, 24^3 144 us
+// and 20^3 183 us; with 4 spills, 226 and 223 us); at p=2 a bound changes nothing and at p=6 it is
+// slower (16^3, 3: 264 us, the compiler's two waves 247 us), so those keep the compiler's choice.
 template <int D, int N, typename T> constexpr int line_waves()
 {
-    if constexpr (D == 3 && N >= 4 && N <= 6 && std::is_same<T, double>::value) return 3;
+    if constexpr (D == 3 && N == 4) return 4;
+    if constexpr (D == 3 && (N == 5 || N == 6) && std::is_same<T, double>::value) return 3;
     return 0;
 }
-template <int D, int N, typename T, int W, bool BND = false, bool GEN = false>
+template <int D, int N, typename T, int W, bool BND = false, int FORM = FORM_EC>
 __global__ void __launch_bounds__((LineGeoS<D, N, T>::BLOCK)) __attribute__((amdgpu_waves_per_eu(W)))
 line_kernel_wb(StageArgs a, Ops1D ops, PhysConst pc)
 {
-    line_block<D, N, T, line_es_single<D, N, T>(), false, false, BND, false, GEN>(
+    line_block<D, N, T, line_es_single<D, N, T>(), false, LINE_NODES, BND, false, FORM>(
         a, ops, pc, xcd_block() * LineGeoS<D, N, T>::EPB);
 }
 
@@ -991,11 +1134,11 @@ line_kernel_wb(StageArgs a, Ops1D ops, PhysConst pc)
 // curved Navier-Stokes p=5 16^3 611 -> 246 us (with the 66 us lifted gradient), Navier-Stokes
 // p=5 16^3 stage 264 -> 160 us.  The metric columns are read from memory by the one item that uses
 // them, so the block's LDS is that of the box.
-template <int D, int N, bool V, bool CV>
+template <int D, int N, bool V, bool CV, int FORM>
 __global__ void __launch_bounds__((LineGeoK<D, N, double, V>::BLOCK)) __attribute__((amdgpu_waves_per_eu(line64_waves<D, N, V, CV>())))
 line64_kernel(StageArgs a, Ops1D ops, PhysConst pc)
 {
-    line_block<D, N, double, line_es<D, N, double, V>(), V, false, false, CV>(
+    line_block<D, N, double, line_es<D, N, double, V>(), V, LINE_NODES, false, CV, FORM>(
         a, ops, pc, xcd_block() * LineGeoK<D, N, double, V>::EPB);
 }
 
@@ -1023,23 +1166,23 @@ line_kernel_ns_w4(StageArgs a, Ops1D ops, PhysConst pc)
 struct BatchBlock {
     int inst, blk0;
 };
-template <int D, int N, typename T, int ES, bool XJ, bool GEN>
+template <int D, int N, typename T, int ES, int XJ, bool GEN>
 __global__ void __launch_bounds__((LineGeo<D, N, T, ES, false, XJ>::BLOCK))
 line_kernel_batch(const BatchBlock *__restrict__ blocks, const StageArgs *__restrict__ args,
                   const PhysConst *__restrict__ pcs, Ops1D ops)
 {
     const BatchBlock bb = blocks[xcd_block()];
-    line_block<D, N, T, ES, false, XJ, false, false, GEN>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
+    line_block<D, N, T, ES, false, XJ, false, false, GEN ? FORM_GEN : FORM_EC>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
 }
 // The same held to W waves/SIMD (amdgpu_waves_per_eu): a candidate tile of the batched
 // autotuner.
-template <int D, int N, typename T, int ES, int W, bool XJ, bool GEN>
+template <int D, int N, typename T, int ES, int W, int XJ, bool GEN>
 __global__ void __launch_bounds__((LineGeo<D, N, T, ES, false, XJ>::BLOCK)) __attribute__((amdgpu_waves_per_eu(W)))
 line_kernel_batch_wb(const BatchBlock *__restrict__ blocks, const StageArgs *__restrict__ args,
                      const PhysConst *__restrict__ pcs, Ops1D ops)
 {
     const BatchBlock bb = blocks[xcd_block()];
-    line_block<D, N, T, ES, false, XJ, false, false, GEN>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
+    line_block<D, N, T, ES, false, XJ, false, false, GEN ? FORM_GEN : FORM_EC>(args[bb.inst], ops, pcs[bb.inst], bb.blk0);
 }
 
 // Tiles the batched autotuner times per (dim, nodes per direction, precision): elements per
@@ -1048,17 +1191,20 @@ line_kernel_batch_wb(const BatchBlock *__restrict__ blocks, const StageArgs *__r
 // occupancy) x threads per block (one per node, or one per line-phase item: XJ).  None changes
 // the arithmetic of an element (the line split LS is fixed per shape for that reason: it
 // reorders the pair sums), so every tile gives the single solve's bits.
+// The last tile is the small meshes' (line_es_small), which the server also takes for groups that do
+// not fill the chip.
 struct BatchTile {
-    int es, waves;
-    bool xj;
+    int es, waves, xj;
 };
-constexpr int BATCH_TILES_2D = 12, BATCH_TILES_3D = 2;
+constexpr int BATCH_TILES_2D = 13, BATCH_TILES_3D = 3;
 constexpr int batch_tile_count(int dim) { return dim == 2 ? BATCH_TILES_2D : BATCH_TILES_3D; }
+constexpr int batch_tile_small(int dim) { return batch_tile_count(dim) - 1; }
 constexpr int batch_waves(int dim, bool fast) { return dim == 2 ? (fast ? 5 : 4) : 0; }
-constexpr BatchTile batch_tile(int dim, bool fast, int v)
+template <int D, int N> constexpr BatchTile batch_tile(bool fast, int v)
 {
+    if (v == batch_tile_small(D)) return BatchTile{line_es_small<D, N>(), 0, LINE_WAVES};
     const int es = (v % 3 == 0) ? 1 : (v % 3 == 1 ? 2 : -2);
-    return BatchTile{es, (v / 3) % 2 ? batch_waves(dim, fast) : 0, v >= 6};
+    return BatchTile{es, (v / 3) % 2 ? batch_waves(D, fast) : 0, v >= 6 ? LINE_ITEMS : LINE_NODES};
 }
 
 } // namespace dgx
