@@ -32,7 +32,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
-KERNEL = {"fp64": "line_kernel_wb<3,4,double,3>", "mixed": "line_kernel<3,4,float>"}
+KERNEL = {"fp64": "line_kernel_wb<3,4,double,4>", "mixed": "line_kernel_wb<3,4,float,4>"}
 TRAFFIC_FILE = {"fp64": os.path.join(ROOT, "profiles", "line_kernel_fp64_tgv_p3_32cubed_traffic.txt"),
                 "mixed": os.path.join(ROOT, "profiles", "line_kernel_mixed_tgv_p3_32cubed_traffic.txt")}
 

@@ -21,8 +21,7 @@
 // The FP64 path's VALU issue is what its stage kernels spend most of their time on, so its
 // versions (the *64 functions) are arranged for fewer instructions than the float ones: one
 // reciprocal serves both 1/(rho1+rho2) and 1/(b1+b2), 1/F_rho comes from its expansion and one
-// Newton step, |avg v|^2 - avg |v|^2 / 2 is v1.v2 / 2, and a node's 1/rho and 1/p come from one
-// reciprocal.  Every sum over the two sides is written so that exchanging them and turning the
+// Newton step, and |avg v|^2 - avg |v|^2 / 2 is v1.v2 / 2.  Every sum over the two sides is written so that exchanging them and turning the
 // normal around gives the exact negative, so a face evaluated from either side needs no
 // selection of an owner.  They take a direction K or (CV) a normal / cofactor column nv.
 #pragma once
@@ -120,20 +119,21 @@ template <typename T> __device__ __forceinline__ FastConst<T> fast_const(const P
 }
 
 // Fills every field of q from q.u; beta is rho/(2p) (Chandrashekar) or rho/p (Ranocha).  In double
-// 1/rho and 1/p = (g-1)^-1 rho / e, e = rho E - |m|^2/2, come from one reciprocal 1/(rho e), and
-// |v|^2, which the FP64 fluxes do not use, is left out.
+// |v|^2, which the FP64 fluxes do not use, is left out.  (One reciprocal 1/(rho e), e = rho E -
+// |m|^2/2, for both 1/rho and 1/p took three operations less and left p three times further off; the
+// pressure's rounding is what a residual at low Mach number is made of.)
 template <typename T, int D>
 __device__ __forceinline__ void node_fill(NodeC<T, D> &q, const FastConst<T> &fc)
 {
     if constexpr (std::is_same<T, double>::value) {
-        double m2 = q.u[1] * q.u[1];
-        for (int k = 1; k < D; ++k) m2 += q.u[1 + k] * q.u[1 + k];
-        const double e = q.u[0] * q.u[D + 1] - 0.5 * m2;
-        const double r = frcp<double>(q.u[0] * e);
-        const double ir = r * e;
-        for (int k = 0; k < D; ++k) q.vel[k] = q.u[1 + k] * ir;
-        q.p = fc.gamm1 * (e * ir);
-        const double rp = fc.inv_gamm1 * (q.u[0] * q.u[0]) * (q.u[0] * r);
+        const double ir = frcp<double>(q.u[0]);
+        double v2 = 0.0;
+        for (int k = 0; k < D; ++k) {
+            q.vel[k] = q.u[1 + k] * ir;
+            v2 += q.vel[k] * q.vel[k];
+        }
+        q.p = fc.gamm1 * (q.u[D + 1] - 0.5 * q.u[0] * v2);
+        const double rp = q.u[0] * frcp<double>(q.p);
         q.b = (fc.two_point == 3) ? rp : 0.5 * rp;
         q.sr = fsqrt<double>(q.u[0]);
         q.c = fsqrt<double>(fc.gam * q.p * ir);
@@ -207,7 +207,8 @@ __device__ __forceinline__ void ec_flux64(const NodeC<double, D> &a, const NodeC
     const bool ra = (fc.two_point == 3);
     const double sr = a.u[0] + b.u[0], sb = a.b + b.b;
     const double t = frcp<double>(sr * sb);
-    const double isr = t * sb, isb = t * sr;
+    // 1/(b1+b2) carries the pressure: one more Newton step takes the products' rounding out again
+    const double isr = t * sb, isb0 = t * sr, isb = isb0 + isb0 * (1.0 - sb * isb0);
     const double fr = (a.u[0] - b.u[0]) * isr, fb = (a.b - b.b) * isb;
     const double ur = fr * fr, ub = fb * fb;
     double Fr = 1.0 + ur * (1.0 / 3.0 + ur * (1.0 / 5.0 + ur * (1.0 / 7.0)));
@@ -462,7 +463,8 @@ __device__ __forceinline__ void roe64(const NodeC<double, D> &L, const NodeC<dou
 // Numerical flux in double along the unit normal n (CV) or sgn e_K, outward of side L; exchanging
 // the sides and turning the normal around gives the exact negative.  GEN: the two-point flux is
 // Kennedy-Gruber or Ismail-Roe, else Chandrashekar or Ranocha; `first` orders the sides for the
-// former, which are not written that way.
+// former, which are not written that way.  Lax-Friedrichs dissipation reads the energies u[D + 1] as
+// well (rebuilt from H they would leave a jump of their rounding times the sound speed).
 template <int D, int K, bool CV, bool GEN>
 __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const NodeC<double, D> &R, double sgn,
                                            const double *n, bool first, const FastConst<double> &fc,
@@ -520,8 +522,7 @@ __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const Node
             const double a = L.u[0] * L.vel[k], b = R.u[0] * R.vel[k];
             out[1 + k] -= hl * (b - a);
         }
-        const double a = L.u[0] * L.h - L.p, b = R.u[0] * R.h - R.p;
-        out[D + 1] -= hl * (b - a);
+        out[D + 1] -= hl * (R.u[D + 1] - L.u[D + 1]);
     }
     if (cf == 1 || cf == 5) roe64<D, K, CV>(L, R, sgn, n, vnL, vnR, fc, out);
 }

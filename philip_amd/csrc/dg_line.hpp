@@ -535,6 +535,11 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
         node_fill<double, D>(qn, fc);
     }
+    if (pc.conv_flux == 0 || pc.conv_flux == 4 || (V && pc.diss_flux == 0)) {
+        // the jump of the energy itself (Lax-Friedrichs, SIPG), which the node cache does not hold
+        qi.u[D + 1] = a.u[((long)e * NS + D + 1) * NP + fi];
+        if (nbl >= 0) qn.u[D + 1] = a.u[((long)nb * NS + D + 1) * NP + fj];
+    }
     double fs[NS];
     num_flux64<D, K, CV, FORM == FORM_GEN>(qi, qn, sgn, nh, own, fc, pc, fs);
     const double iwb = ops.inv_wb;
@@ -601,8 +606,7 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
                 const double ma = qi.u[0] * qi.vel[k], mb = qn.u[0] * qn.vel[k];
                 du[1 + k] = ma - mb;
             }
-            const double ea = qi.u[0] * qi.h - qi.p, eb = qn.u[0] * qn.h - qn.p;
-            du[D + 1] = ea - eb;
+            du[D + 1] = qi.u[D + 1] - qn.u[D + 1];
             viscous_jump64<D>(qi, du, nh, pc, ja);
             viscous_jump64<D>(qn, du, nh, pc, jb);
             double pen = a.penalty;
