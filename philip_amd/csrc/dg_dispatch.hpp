@@ -24,11 +24,32 @@ inline int check_launch(dgx_ctx *c, const char *what)
     return DGX_OK;
 }
 
+// The small meshes' block of the line kernel, if the mesh is one; tells whether it was launched.
+// A mesh of at most a block per compute unit is bound by the length of one block's chain, not by
+// throughput.  Right-hand side, default -> small, at 0.4 blocks per unit: FP64 2D p=2 7.6 -> 5.6
+// us, p=4 9.6 -> 5.9, p=6 11.1 -> 7.9; 3D p=1 10.6 -> 6.0, p=3 10.0 -> 6.1, p=5 12.2 -> 8.2; mixed 3D
+// p=3 10.3 -> 6.2.  At one block per unit they meet (3D p=2 10.0 and 10.1, p=4 11.7 and 12.0); with
+// 1.5 the small blocks are slower.  FP64 p=6 in 3D would spill.
+template <int D, int N, typename T, int FORM>
+bool line_small_dn(dgx_ctx *c, const StageArgs &a)
+{
+    if constexpr (FORM != FORM_GEN && !(D == 3 && N == 7 && std::is_same<T, double>::value)) {
+        using LS = LineGeoSmall<D, N, T>;
+        constexpr int EPB = LineGeoS<D, N, T>::EPB;
+        if (c->has_boundary || (c->ncells + EPB - 1) / EPB > c->n_cu) return false;
+        hipLaunchKernelGGL((line_kernel_small<D, N, T, FORM>), dim3((c->ncells + LS::EPB - 1) / LS::EPB),
+                           dim3(LS::BLOCK), 0, c->stream, a, c->ops, c->pc);
+        return true;
+    }
+    return false;
+}
+
 // Euler on the box in the line kernel, with boundary faces or without.
 template <int D, int N, typename T, int FORM>
 void line_dn(dgx_ctx *c, const StageArgs &a)
 {
     using LG = LineGeoS<D, N, T>;
+    if (line_small_dn<D, N, T, FORM>(c, a)) return;
     auto go = [&](auto bc) {
         constexpr bool BND = decltype(bc)::value;
         const dim3 grid((c->ncells + LG::EPB - 1) / LG::EPB), block(LG::BLOCK);
@@ -38,26 +59,14 @@ void line_dn(dgx_ctx *c, const StageArgs &a)
         else
             hipLaunchKernelGGL((line_kernel<D, N, T, BND, FORM>), grid, block, 0, c->stream, a, c->ops, c->pc);
     };
-    if (c->has_boundary) {
-        go(std::true_type{});
-        return;
-    }
-    // A mesh of at most a block per compute unit is bound by the length of one block's chain, not by
-    // throughput.  Right-hand side, default -> small, at 0.4 blocks per unit: FP64 2D p=2 7.6 -> 5.6
-    // us, p=4 9.6 -> 5.9, p=6 11.1 -> 7.9; 3D p=1 10.6 -> 6.0, p=3 10.0 -> 6.1, p=5 12.2 -> 8.2; mixed 3D
-    // p=3 10.3 -> 6.2.  At one block per unit they meet (3D p=2 10.0 and 10.1, p=4 11.7 and 12.0); with
-    // 1.5 the small blocks are slower.  FP64 p=6 would spill.
-    if constexpr (FORM != FORM_GEN && !(D == 3 && N == 7 && std::is_same<T, double>::value)) {
-        using LS = LineGeoSmall<D, N, T>;
-        const int blocks = (c->ncells + LG::EPB - 1) / LG::EPB;
-        if (blocks <= c->n_cu) {
-            hipLaunchKernelGGL((line_kernel_small<D, N, T, FORM>), dim3((c->ncells + LS::EPB - 1) / LS::EPB),
-                               dim3(LS::BLOCK), 0, c->stream, a, c->ops, c->pc);
-            return;
-        }
-    }
-    go(std::false_type{});
+    if (c->has_boundary) go(std::true_type{});
+    else go(std::false_type{});
 }
+
+// FP64 conservative form on the box: the line kernel in 3D up to p=5 (rhs of 28^3 p=3 67 -> 54 us, 16^3
+// p=5 51 -> 42 us); in 2D (300^2 p=4 62 against 67 us) and at p=6 (14^3 71 against 77 us) stage2_kernel,
+// small meshes apart.
+template <int D, int N> constexpr bool line_conservative() { return D == 3 && N <= 6; }
 
 // Stage kernel of a context.  FP64: the line kernel, but for walls with the viscous terms, boundary
 // faces on a curvilinear grid, and Kennedy-Gruber or Ismail-Roe fluxes with the viscous terms or on a
@@ -71,8 +80,12 @@ void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
     const bool nsv = D == 3 && c->P.pde == DGX_NAVIER_STOKES;
     if (!nsv && !curv) {
         if constexpr (FP64) {
-            if (!split) return line_dn<D, N, T, FORM_CONS>(c, a);
-            if (c->pc.two_point < 2) return line_dn<D, N, T, FORM_GEN>(c, a);
+            if constexpr (line_conservative<D, N>()) {
+                if (!split) return line_dn<D, N, T, FORM_CONS>(c, a);
+            } else {
+                if (!split && line_small_dn<D, N, T, FORM_CONS>(c, a)) return;
+            }
+            if (split && c->pc.two_point < 2) return line_dn<D, N, T, FORM_GEN>(c, a);
         }
         if (split) return line_dn<D, N, T, FORM_EC>(c, a);
     }
@@ -139,7 +152,7 @@ void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
         else go2(no, no, yes, yes);
         return;
     }
-    if constexpr (!FP64) {  // conservative Euler on the box
+    if constexpr (!FP64 || !line_conservative<D, N>()) {  // conservative Euler on the box
         if (bnd) go2(no, no, yes, no);
         else go2(no, no, no, no);
     }

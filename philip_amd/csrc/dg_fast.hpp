@@ -370,18 +370,17 @@ __device__ __forceinline__ void roe_fast(const NodeC<T, D> &L, const NodeC<T, D>
     for (int s = 0; s < D + 2; ++s) out[s] = T(-0.5) * A[s];
 }
 
-// Convective flux of a cached node along e_K or (CV) contracted with nv.
+// Convective flux of a node (with its momentum) along e_K or (CV) contracted with nv.
 template <int D, int K, bool CV>
 __device__ __forceinline__ void convective_flux64(const NodeC<double, D> &q, const double *nv, double *f)
 {
-    double vn;
+    double m;
     if constexpr (CV) {
-        vn = q.vel[0] * nv[0];
-        for (int k = 1; k < D; ++k) vn += q.vel[k] * nv[k];
+        m = q.u[1] * nv[0];
+        for (int k = 1; k < D; ++k) m += q.u[1 + k] * nv[k];
     } else {
-        vn = q.vel[K];
+        m = q.u[1 + K];
     }
-    const double m = q.u[0] * vn;
     f[0] = m;
     for (int k = 0; k < D; ++k) {
         f[1 + k] = m * q.vel[k];
@@ -464,8 +463,9 @@ __device__ __forceinline__ void roe64(const NodeC<double, D> &L, const NodeC<dou
 // the sides and turning the normal around gives the exact negative.  GEN: the two-point flux is
 // Kennedy-Gruber or Ismail-Roe, else Chandrashekar or Ranocha; `first` orders the sides for the
 // former, which are not written that way.  Lax-Friedrichs dissipation reads the energies u[D + 1] as
-// well (rebuilt from H they would leave a jump of their rounding times the sound speed).
-template <int D, int K, bool CV, bool GEN>
+// well (rebuilt from H they would leave a jump of their rounding times the sound speed).  MOM: the
+// nodes hold their momentum, else it is rho v.
+template <int D, int K, bool CV, bool GEN, bool MOM = false>
 __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const NodeC<double, D> &R, double sgn,
                                            const double *n, bool first, const FastConst<double> &fc,
                                            const PhysConst &pc, double *out)
@@ -504,7 +504,19 @@ __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const Node
         if constexpr (!CV)
             for (int s = 0; s < D + 2; ++s) out[s] *= sgn;
     } else {
-        const double mL = L.u[0] * vnL, mR = R.u[0] * vnR, ps = 0.5 * (L.p + R.p);
+        double mL = L.u[0] * vnL, mR = R.u[0] * vnR;
+        if constexpr (MOM && CV) {
+            mL = L.u[1] * n[0];
+            mR = R.u[1] * n[0];
+            for (int k = 1; k < D; ++k) {
+                mL += L.u[1 + k] * n[k];
+                mR += R.u[1 + k] * n[k];
+            }
+        } else if constexpr (MOM) {
+            mL = L.u[1 + K] * sgn;
+            mR = R.u[1 + K] * sgn;
+        }
+        const double ps = 0.5 * (L.p + R.p);
         out[0] = 0.5 * (mL + mR);
         for (int k = 0; k < D; ++k) {
             const double a = mL * L.vel[k], b = mR * R.vel[k];
@@ -519,7 +531,11 @@ __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const Node
         const double hl = 0.5 * fmx<double>(fab<double>(vnL) + L.c, fab<double>(vnR) + R.c);
         out[0] -= hl * (R.u[0] - L.u[0]);
         for (int k = 0; k < D; ++k) {
-            const double a = L.u[0] * L.vel[k], b = R.u[0] * R.vel[k];
+            double a = L.u[0] * L.vel[k], b = R.u[0] * R.vel[k];
+            if (MOM) {
+                a = L.u[1 + k];
+                b = R.u[1 + k];
+            }
             out[1 + k] -= hl * (b - a);
         }
         out[D + 1] -= hl * (R.u[D + 1] - L.u[D + 1]);

@@ -203,6 +203,21 @@ template <int D> __device__ __forceinline__ void nodef_load_pair(const double *q
     n.b = q[(D + 2) * st];
 }
 
+// FP64, conservative form: the cache holds the momentum in the velocity's place and 1/rho in beta's,
+// so that the mass flux is the momentum itself, as it is in a trace.
+template <int D> __device__ __forceinline__ void nodef_to_momentum(NodeC<double, D> &n)
+{
+    for (int k = 0; k < D; ++k) n.vel[k] = n.u[1 + k];
+    n.b = frcp<double>(n.u[0]);
+}
+template <int D> __device__ __forceinline__ void nodef_from_momentum(NodeC<double, D> &n)
+{
+    for (int k = 0; k < D; ++k) {
+        n.u[1 + k] = n.vel[k];
+        n.vel[k] = n.u[1 + k] * n.b;
+    }
+}
+
 template <typename T, int D>
 __device__ __forceinline__ void nodef_load(const T *q, int st, NodeC<T, D> &n)
 {
@@ -358,6 +373,7 @@ __device__ __forceinline__ void cons_line64(const Ops1D &ops, const double *sq, 
         NodeC<double, D> B;
         double f[NS];
         nodef_load_pair<D>(q, NP, B);
+        nodef_from_momentum<D>(B);
         B.h = q[(D + 3) * NP];
         convective_flux64<D, K, CV>(B, cm[CV ? b : 0], f);
 #pragma unroll
@@ -529,8 +545,10 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
     }
     NodeC<double, D> qi, qn;
     nodef_load<double, D>(in.sq + le * LG::ESQ + qpos<D, N>(fi), NP, qi);
+    if constexpr (FORM == FORM_CONS) nodef_from_momentum<D>(qi);
     if (nbl >= 0) {
         nodef_load<double, D>(in.sq + nbl * LG::ESQ + qpos<D, N>(fj), NP, qn);
+        if constexpr (FORM == FORM_CONS) nodef_from_momentum<D>(qn);
     } else {
         for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
         node_fill<double, D>(qn, fc);
@@ -541,7 +559,7 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         if (nbl >= 0) qn.u[D + 1] = a.u[((long)nb * NS + D + 1) * NP + fj];
     }
     double fs[NS];
-    num_flux64<D, K, CV, FORM == FORM_GEN>(qi, qn, sgn, nh, own, fc, pc, fs);
+    num_flux64<D, K, CV, FORM == FORM_GEN, FORM == FORM_CONS>(qi, qn, sgn, nh, own, fc, pc, fs);
     const double iwb = ops.inv_wb;
     const double w = CV ? iwb * area : iwb;
     for (int s = 0; s < NS; ++s) {
@@ -715,6 +733,7 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
         for (int s = 0; s < NS; ++s) n.u[s] = T(ud[s]);
         node_fill<T, D>(n, fc);
         flag_nonphysical<T>(a, n.u[0], n.p);
+        if constexpr (FORM == FORM_CONS) nodef_to_momentum<D>(n);
         nodef_store<T, D>(sQ + le * LG::ESQ + qpos<D, N>(i), NP, n);
     }
 #pragma unroll
