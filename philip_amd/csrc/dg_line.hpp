@@ -695,7 +695,9 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
     if (active)
         for (int s = 0; s < NS; ++s) ud[s] = a.u[((long)e * NS + s) * NP + i];
     double pf2[NS], pf3[NS];
-    constexpr bool PREFETCH = FAST ? LINE_PREFETCH_RK_F : LINE_PREFETCH_RK_D;
+    // mixed 3D p=6: like FP64, its registers are read after the line phase (loaded first it spills)
+    constexpr bool EARLY = FAST && (V || D == 2 || N != 7);
+    constexpr bool PREFETCH = EARLY ? LINE_PREFETCH_RK_F : LINE_PREFETCH_RK_D;
     const bool pf = PREFETCH && active && a.mode == MODE_LSRK && !a.lsrk_first;
     if (pf)
         for (int s = 0; s < NS; ++s) {
@@ -1015,16 +1017,16 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
     }
     __syncthreads();  // node cache and traces consumed; their storage now takes the partials
     // FP64: the registers of the epilogue are read from here on; mixed: those of a Butcher stage (S2
-    // and S3 were loaded in phase A; not at p=6 in 3D, which spills; 2D p=3 512^2 RK4 stage 157 -> 128 us, Navier-Stokes p=5 16^3 147 ->
+    // and S3 were loaded in phase A; 2D p=3 512^2 RK4 stage 157 -> 128 us, Navier-Stokes p=5 16^3 147 ->
     // 129 us with the lifted gradient)
-    constexpr bool LATE_PF = FAST ? (V || D == 2 || N != 7) : line_late_prefetch_d<D, N>();
+    constexpr bool LATE_PF = FAST || line_late_prefetch_d<D, N>();
     const bool late_pf = LATE_PF && active &&
-                         ((!FAST && a.mode == MODE_LSRK && !a.lsrk_first) || a.mode == MODE_BUTCHER);
+                         ((!EARLY && a.mode == MODE_LSRK && !a.lsrk_first) || a.mode == MODE_BUTCHER);
     // FP64 at N >= 4: the stage state is read again here for the epilogue (an L2 hit: the block
     // read it in phase A) instead of being held in registers through the line phase (TGV 32^3
     // p=3: 177 -> 170 us per stage, 64 -> 16 B/lane of spills; p=4 24^3 294 -> 244 us; at p=2
     // slower)
-    constexpr bool REREAD = !FAST && LATE_PF && N >= 4;
+    constexpr bool REREAD = !EARLY && LATE_PF && N >= 4;
     double ue[NS];
     if (REREAD && active && a.mode == MODE_LSRK)
         for (int s = 0; s < NS; ++s) ue[s] = a.u[((long)e * NS + s) * NP + i];
