@@ -10,6 +10,7 @@
 
 #include "dg_host.hpp"
 #include "dg_line.hpp"
+#include "dg_rules.hpp"
 #include "dg_stage2.hpp"
 
 namespace dgx {
@@ -73,11 +74,13 @@ template <int D, int N> constexpr bool line_conservative() { return D == 3 && N 
 // curvilinear grid, which are stage2_kernel's.  Mixed: the line kernel for the periodic split form and
 // for Euler boundary faces on the box, stage2_kernel for the rest.
 template <int D, int N, typename T>
-void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
+void stage2_dn(dgx_ctx *c, StageArgs a, dim3 grid, dim3 block)
 {
     constexpr bool FP64 = std::is_same<T, double>::value;
     const bool split = c->P.use_split_form != 0, bnd = c->has_boundary, curv = c->curv;
     const bool nsv = D == 3 && c->P.pde == DGX_NAVIER_STOKES;
+    const double mb = 1e-6 * sizeof(double) * c->ncells * Geo<D, N>::NS * Geo<D, N>::NP;
+    a.s1_cached = store_stays_cached(D, N, true, curv, mb);
     if (!nsv && !curv) {
         if constexpr (FP64) {
             if constexpr (line_conservative<D, N>()) {
@@ -122,6 +125,7 @@ void stage2_dn(dgx_ctx *c, const StageArgs &a, dim3 grid, dim3 block)
             return;
         }
     }
+    a.s1_cached = store_stays_cached(D, N, false, curv, mb);
     auto go2 = [&](auto sc, auto vc, auto bc, auto cc) {
         hipLaunchKernelGGL((stage2_kernel<D, N, decltype(sc)::value, decltype(vc)::value, T, decltype(bc)::value,
                                           decltype(cc)::value>),

@@ -48,6 +48,7 @@ struct StageArgs {
     // low-storage RK 3S* (S1 ping-pong, S2 in place, S3 = u_n, S4 optional)
     double *s1_out, *s2, *s3, *s4;
     int lsrk_first;           // stage 0: S2 = delta*S1, S3 = S1 written
+    int s1_cached;            // s1_out stored to stay in the caches (store_stays_cached), else streamed
     double delta, g0, g1, g2, beta, bhat, dt;
     // Butcher explicit RK
     const double *u0;         // u_n
@@ -129,7 +130,7 @@ __device__ __forceinline__ int node_with(int i, int k, int l)
 // Streaming access to the RK registers: each value is read or written once per
 // stage and the registers together exceed the caches, so the stage kernels
 // mark these accesses non-temporal (STREAM_NT) to keep L2 for the neighbour
-// face traces, but for the store of the next stage's state (stage_epilogue).
+// face traces, but for the store of the next stage's state where store_stays_cached.
 constexpr bool STREAM_NT = true;
 __device__ __forceinline__ double ld_stream(const double *p)
 {
@@ -140,6 +141,12 @@ __device__ __forceinline__ void st_stream(double *p, double v)
 {
     if constexpr (STREAM_NT) __builtin_nontemporal_store(v, p);
     else *p = v;
+}
+// The ordinary store, as an atomic of no ordering: on the two sides of a branch an ordinary store and
+// st_stream of the same value to the same address are merged into one, without the streaming hint.
+__device__ __forceinline__ void st_cached(double *p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
 }
 
 // Phase E of the stage kernels, in FP64: du/dt = acc / h and the output of the
@@ -171,27 +178,28 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &
             a.out[base + s * NP] = a.out[base + s * NP] + a.bhat * r;
         }
     } else if (a.mode == MODE_LSRK) {
+        double n1[NS];
         for (int s = 0; s < NS; ++s) {
             const long idx = base + s * NP;
             const double s1 = ud[s];
             // use_pf: S2, S3 already loaded by the caller into pf2 / pf3 (non-first stages)
             const double s2 = a.lsrk_first ? 0.0 + a.delta * s1 : (use_pf ? pf2[s] : ld_stream(a.s2 + idx)) + a.delta * s1;
             const double s3 = a.lsrk_first ? s1 : (use_pf ? pf3[s] : ld_stream(a.s3 + idx));
-            double n1 = s1 * a.g0;
-            n1 += a.g1 * s2;
-            n1 += a.g2 * s3;
+            n1[s] = s1 * a.g0;
+            n1[s] += a.g1 * s2;
+            n1[s] += a.g2 * s3;
             const double r = dudt[s] * a.dt;
-            n1 += a.beta * r;
+            n1[s] += a.beta * r;
             st_stream(a.s2 + idx, s2);
             if (a.lsrk_first) st_stream(a.s3 + idx, s1);
-            // the next stage's state: on the box it is stored to stay in the last-level cache for that
-            // stage's read (TGV p=3 32^3 stage, FP64 117 -> 108 us, mixed 98 -> 91.5 us; S2 as well: no
-            // further gain); on a curvilinear grid the metric terms need the cache more (146 us, 154 us
-            // with this store)
-            if (a.met) st_stream(a.s1_out + idx, n1);
-            else a.s1_out[idx] = n1;
             if (a.s4) a.s4[idx] = (a.lsrk_first ? s1 : a.s4[idx]) + a.bhat * r;
         }
+        // the next stage's state, stored to stay in the caches for that stage's read or streamed
+        // (store_stays_cached; S2 cached as well: no further gain)
+        if (a.s1_cached)
+            for (int s = 0; s < NS; ++s) st_cached(a.s1_out + base + s * NP, n1[s]);
+        else
+            for (int s = 0; s < NS; ++s) st_stream(a.s1_out + base + s * NP, n1[s]);
     } else {
         for (int s = 0; s < NS; ++s) {
             const long idx = base + s * NP;

@@ -1,0 +1,48 @@
+"""The rules that choose kernels and store policies (dg_rules.hpp, host build) on both sides of their
+lines, at the sizes where the two sides were measured; and that a store policy is still there after
+the compiler."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("rules") / "rules_host")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-o", exe, os.path.join(HERE, "host", "rules_host.cpp")], check=True)
+
+    def ask(*words):
+        line = " ".join(str(int(w) if isinstance(w, bool) else w) for w in words)
+        return int(subprocess.run([exe], input=line, capture_output=True, text=True, check=True).stdout)
+
+    return ask
+
+
+# dim, p, line kernel, curved, state in MB; faster cached
+STORE = [(3, 3, True, False, 8.6, False), (3, 3, True, False, 84, True), (3, 3, True, False, 119, True),
+         (2, 1, True, False, 3.2, False), (2, 2, False, False, 7.1, True), (2, 1, True, False, 320, True), (3, 3, False, False, 20, False),
+         (3, 2, False, False, 84, True), (3, 6, False, False, 127, False), (2, 3, False, False, 134, False),
+         (2, 1, False, False, 134, True), (3, 3, True, True, 62, True), (3, 3, True, True, 84, False),
+         (3, 1, True, True, 170, True), (3, 4, False, True, 122, False)]
+
+
+@pytest.mark.parametrize("dim,p,line,curved,mb,cached", STORE)
+def test_store_policy(rules, dim, p, line, curved, mb, cached):
+    assert rules("store", dim, p + 1, line, curved, mb) == cached
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
+def test_both_store_policies_are_in_the_code(tmp_path):
+    """The state's four stores once streamed and once not, beside S2's four streamed ones."""
+    out = str(tmp_path / "s.s")
+    subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=on", "-Xclang",
+                    "-target-feature", "-Xclang", "-packed-fp32-ops", "--cuda-device-only", "-S", "-o", out,
+                    os.path.join(HERE, "host", "stage_store.hip")], check=True, capture_output=True)
+    stores = [x for x in open(out).read().splitlines() if re.search(r"\bglobal_store_dwordx2\b", x)]
+    assert sum(" nt" in x for x in stores) == 8 and sum(" nt" not in x for x in stores) == 4
