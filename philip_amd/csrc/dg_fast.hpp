@@ -274,8 +274,38 @@ __device__ __forceinline__ void ec_flux64(const NodeC<double, D> &a, const NodeC
     }
 }
 
-// Kennedy-Gruber and Ismail-Roe of two cached nodes through the generic evaluation of
-// dg_physics.hpp (CV: contracted with nv).
+// Volume form of an FP64 line kernel: Chandrashekar / Ranocha split form, the split form with one of
+// the other two-point fluxes (a kernel of its own: the generic evaluation sets the register count of
+// a kernel that holds both -- p=3: 153 VGPRs, the curved kernel 246), the conservative form.
+enum LineForm { FORM_EC = 0, FORM_GEN = 1, FORM_CONS = 2 };
+
+// What a form keeps in two fields of a node's FP64 cache (rho, v, p, beta, H, c, sqrt(rho)): the
+// conservative form the momentum in the velocity's place and 1/rho in beta's, so that the mass flux is
+// the momentum itself, as it is in a trace; Kennedy-Gruber and Ismail-Roe, which have no beta, E there.
+template <int D, int FORM> __device__ __forceinline__ void node_to_cache64(NodeC<double, D> &n)
+{
+    if constexpr (FORM == FORM_CONS) {
+        for (int k = 0; k < D; ++k) n.vel[k] = n.u[1 + k];
+        n.b = frcp<double>(n.u[0]);
+    } else if constexpr (FORM == FORM_GEN) {
+        n.b = n.u[D + 1];
+    }
+}
+template <int D, int FORM> __device__ __forceinline__ void node_from_cache64(NodeC<double, D> &n)
+{
+    if constexpr (FORM == FORM_CONS) {
+        for (int k = 0; k < D; ++k) {
+            n.u[1 + k] = n.vel[k];
+            n.vel[k] = n.u[1 + k] * n.b;
+        }
+    } else if constexpr (FORM == FORM_GEN) {
+        n.u[D + 1] = n.b;
+    }
+}
+
+// Kennedy-Gruber and Ismail-Roe of two nodes through the generic evaluation of dg_physics.hpp (CV:
+// contracted with nv).  Kennedy-Gruber averages E / rho: E is the node's own (rebuilt as rho H - p its
+// rounding makes the energy flux a fifth less accurate).
 template <int D, int K, bool CV>
 __device__ __forceinline__ void other_flux64(const NodeC<double, D> &a, const NodeC<double, D> &b, const double *nv,
                                              const PhysConst &pc, double *f)
@@ -292,8 +322,8 @@ __device__ __forceinline__ void other_flux64(const NodeC<double, D> &a, const No
     }
     qa.p = a.p;
     qb.p = b.p;
-    ua[D + 1] = a.u[0] * a.h - a.p;
-    ub[D + 1] = b.u[0] * b.h - b.p;
+    ua[D + 1] = a.u[D + 1];
+    ub[D + 1] = b.u[D + 1];
     if constexpr (CV) two_point_flux_vec<double, D>(ua, qa, ub, qb, nv, pc, f);
     else two_point_flux_dir<double, D>(ua, qa, ub, qb, K, pc, f);
 }
@@ -497,8 +527,8 @@ __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const Node
             }
             a.p = first ? L.p : R.p;
             b.p = first ? R.p : L.p;
-            a.h = first ? L.h : R.h;
-            b.h = first ? R.h : L.h;
+            a.u[D + 1] = first ? L.u[D + 1] : R.u[D + 1];
+            b.u[D + 1] = first ? R.u[D + 1] : L.u[D + 1];
             other_flux64<D, K, CV>(a, b, n, pc, out);
         }
         if constexpr (!CV)

@@ -118,11 +118,6 @@ template <int D, int N, typename T, int ES = 1, bool V = false, int XJ = LINE_NO
     static constexpr int SBUF = EPB * ESN + ((ESQ + ESFV + ESNV > ESV) ? EPB * (ESQ + ESFV + ESNV) : EPB * ESV);
 };
 
-// Volume form of an FP64 line kernel: Chandrashekar / Ranocha split form, the split form with one of
-// the other two-point fluxes (a kernel of its own: the generic evaluation sets the register count of
-// a kernel that holds both -- p=3: 153 VGPRs, the curved kernel 246), the conservative form.
-enum LineForm { FORM_EC = 0, FORM_GEN = 1, FORM_CONS = 2 };
-
 // Elements-per-block variant of the single-solve line kernel: 1 for Euler; for
 // Navier-Stokes (V) the 256-node default block halved until its LDS fits 64 KB
 // (down to one element).
@@ -201,21 +196,6 @@ template <int D> __device__ __forceinline__ void nodef_load_pair(const double *q
     for (int k = 0; k < D; ++k) n.vel[k] = q[(1 + k) * st];
     n.p = q[(D + 1) * st];
     n.b = q[(D + 2) * st];
-}
-
-// FP64, conservative form: the cache holds the momentum in the velocity's place and 1/rho in beta's,
-// so that the mass flux is the momentum itself, as it is in a trace.
-template <int D> __device__ __forceinline__ void nodef_to_momentum(NodeC<double, D> &n)
-{
-    for (int k = 0; k < D; ++k) n.vel[k] = n.u[1 + k];
-    n.b = frcp<double>(n.u[0]);
-}
-template <int D> __device__ __forceinline__ void nodef_from_momentum(NodeC<double, D> &n)
-{
-    for (int k = 0; k < D; ++k) {
-        n.u[1 + k] = n.vel[k];
-        n.vel[k] = n.u[1 + k] * n.b;
-    }
 }
 
 template <typename T, int D>
@@ -316,10 +296,8 @@ __device__ __forceinline__ void pairs64(const Ops1D &ops, const PhysConst &pc, c
             if constexpr (!GEN) {
                 ec_flux64<D, K, CV>(A, B, nv, fc, F);
             } else {
-                const double *qa = sq + qpos<D, N>(line_node<D, N>(K, line, p0)) + (D + 3) * NP;
-                const double *qb = sq + qpos<D, N>(line_node<D, N>(K, line, p1)) + (D + 3) * NP;
-                A.h = qa[0];
-                B.h = qb[0];
+                node_from_cache64<D, FORM_GEN>(A);
+                node_from_cache64<D, FORM_GEN>(B);
                 other_flux64<D, K, CV>(A, B, nv, pc, F);
             }
             const double s01 = ops.Sk[p0][p1], s10 = ops.Sk[p1][p0];
@@ -373,7 +351,7 @@ __device__ __forceinline__ void cons_line64(const Ops1D &ops, const double *sq, 
         NodeC<double, D> B;
         double f[NS];
         nodef_load_pair<D>(q, NP, B);
-        nodef_from_momentum<D>(B);
+        node_from_cache64<D, FORM_CONS>(B);
         B.h = q[(D + 3) * NP];
         convective_flux64<D, K, CV>(B, cm[CV ? b : 0], f);
 #pragma unroll
@@ -545,15 +523,15 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
     }
     NodeC<double, D> qi, qn;
     nodef_load<double, D>(in.sq + le * LG::ESQ + qpos<D, N>(fi), NP, qi);
-    if constexpr (FORM == FORM_CONS) nodef_from_momentum<D>(qi);
+    node_from_cache64<D, FORM>(qi);
     if (nbl >= 0) {
         nodef_load<double, D>(in.sq + nbl * LG::ESQ + qpos<D, N>(fj), NP, qn);
-        if constexpr (FORM == FORM_CONS) nodef_from_momentum<D>(qn);
+        node_from_cache64<D, FORM>(qn);
     } else {
         for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
         node_fill<double, D>(qn, fc);
     }
-    if (pc.conv_flux == 0 || pc.conv_flux == 4 || (V && pc.diss_flux == 0)) {
+    if (FORM != FORM_GEN && (pc.conv_flux == 0 || pc.conv_flux == 4 || (V && pc.diss_flux == 0))) {
         // the jump of the energy itself (Lax-Friedrichs, SIPG), which the node cache does not hold
         qi.u[D + 1] = a.u[((long)e * NS + D + 1) * NP + fi];
         if (nbl >= 0) qn.u[D + 1] = a.u[((long)nb * NS + D + 1) * NP + fj];
@@ -735,7 +713,7 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
         for (int s = 0; s < NS; ++s) n.u[s] = T(ud[s]);
         node_fill<T, D>(n, fc);
         flag_nonphysical<T>(a, n.u[0], n.p);
-        if constexpr (FORM == FORM_CONS) nodef_to_momentum<D>(n);
+        if constexpr (!FAST) node_to_cache64<D, FORM>(n);
         nodef_store<T, D>(sQ + le * LG::ESQ + qpos<D, N>(i), NP, n);
     }
 #pragma unroll
