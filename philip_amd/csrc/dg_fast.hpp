@@ -282,8 +282,14 @@ enum LineForm { FORM_EC = 0, FORM_GEN = 1, FORM_CONS = 2 };
 // What a form keeps in two fields of a node's FP64 cache (rho, v, p, beta, H, c, sqrt(rho)): the
 // conservative form the momentum in the velocity's place and 1/rho in beta's, so that the mass flux is
 // the momentum itself, as it is in a trace; Kennedy-Gruber and Ismail-Roe, which have no beta, E there.
-template <int D, int FORM> __device__ __forceinline__ void node_to_cache64(NodeC<double, D> &n)
+// Lax-Friedrichs dissipation, which does not read sqrt(rho), has E in that field in every form
+// (energy_in_sr): read from memory by the face items instead, E was a round trip in the middle of the
+// line phase (conservative rhs 3D p=3 small mesh 5.9 -> 6.4 us, default block p=5 7.9 -> 9.9 us).
+__device__ __forceinline__ bool energy_in_sr(int conv_flux) { return conv_flux == 0 || conv_flux == 4; }
+template <int D, int FORM>
+__device__ __forceinline__ void node_to_cache64(const FastConst<double> &fc, NodeC<double, D> &n)
 {
+    if (energy_in_sr(fc.conv_flux)) n.sr = n.u[D + 1];
     if constexpr (FORM == FORM_CONS) {
         for (int k = 0; k < D; ++k) n.vel[k] = n.u[1 + k];
         n.b = frcp<double>(n.u[0]);

@@ -531,8 +531,11 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
         node_fill<double, D>(qn, fc);
     }
-    if (FORM != FORM_GEN && (pc.conv_flux == 0 || pc.conv_flux == 4 || (V && pc.diss_flux == 0))) {
-        // the jump of the energy itself (Lax-Friedrichs, SIPG), which the node cache does not hold
+    // the jump of the energy itself (Lax-Friedrichs, SIPG)
+    if (energy_in_sr(pc.conv_flux)) {
+        qi.u[D + 1] = qi.sr;
+        if (nbl >= 0) qn.u[D + 1] = qn.sr;
+    } else if (V && pc.diss_flux == 0) {
         qi.u[D + 1] = a.u[((long)e * NS + D + 1) * NP + fi];
         if (nbl >= 0) qn.u[D + 1] = a.u[((long)nb * NS + D + 1) * NP + fj];
     }
@@ -713,7 +716,7 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
         for (int s = 0; s < NS; ++s) n.u[s] = T(ud[s]);
         node_fill<T, D>(n, fc);
         flag_nonphysical<T>(a, n.u[0], n.p);
-        if constexpr (!FAST) node_to_cache64<D, FORM>(n);
+        if constexpr (!FAST) node_to_cache64<D, FORM>(fc, n);
         nodef_store<T, D>(sQ + le * LG::ESQ + qpos<D, N>(i), NP, n);
     }
 #pragma unroll

@@ -10,9 +10,9 @@
 using namespace dgx;
 
 // the fields that are stored, and nothing else
-static NodeC<double, 3> cached(NodeC<double, 3> n)
+static NodeC<double, 3> cached(const FastConst<double> &fc, NodeC<double, 3> n)
 {
-    node_to_cache64<3, FORM_GEN>(n);
+    node_to_cache64<3, FORM_GEN>(fc, n);
     NodeC<double, 3> m;
     for (double &x : m.u) x = NAN;
     m.u[0] = n.u[0];
@@ -51,7 +51,7 @@ int main()
         qb.p = b.p;
         double f[3][5];
         other_flux64<3, 0, false>(a, b, nullptr, pc, f[0]);
-        other_flux64<3, 0, false>(cached(a), cached(b), nullptr, pc, f[1]);
+        other_flux64<3, 0, false>(cached(fc, a), cached(fc, b), nullptr, pc, f[1]);
         two_point_flux_dir<double, 3>(a.u, qa, b.u, qb, 0, pc, f[2]);
         for (auto &r : f)
             for (double x : r) printf("%.17e ", x);
