@@ -531,13 +531,16 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
         node_fill<double, D>(qn, fc);
     }
-    // the jump of the energy itself (Lax-Friedrichs, SIPG)
+    // the jump of the energy itself (Lax-Friedrichs, SIPG), and of the momentum itself (SIPG): rebuilt
+    // from the cache, they would leave a jump of their own rounding
     if (energy_in_sr(pc.conv_flux)) {
         qi.u[D + 1] = qi.sr;
         if (nbl >= 0) qn.u[D + 1] = qn.sr;
-    } else if (V && pc.diss_flux == 0) {
-        qi.u[D + 1] = a.u[((long)e * NS + D + 1) * NP + fi];
-        if (nbl >= 0) qn.u[D + 1] = a.u[((long)nb * NS + D + 1) * NP + fj];
+    }
+    if (V && pc.diss_flux == 0) {
+        for (int s = 1; s < NS; ++s) qi.u[s] = a.u[((long)e * NS + s) * NP + fi];
+        if (nbl >= 0)
+            for (int s = 1; s < NS; ++s) qn.u[s] = a.u[((long)nb * NS + s) * NP + fj];
     }
     double fs[NS];
     num_flux64<D, K, CV, FORM == FORM_GEN, FORM == FORM_CONS>(qi, qn, sgn, nh, own, fc, pc, fs);
@@ -600,12 +603,7 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         for (int s = 0; s < NVS; ++s) pj[s] = 0.0;
         if (pc.diss_flux == 0) {
             double du[NS], ja[NVS], jb[NVS];
-            du[0] = qi.u[0] - qn.u[0];
-            for (int k = 0; k < D; ++k) {
-                const double ma = qi.u[0] * qi.vel[k], mb = qn.u[0] * qn.vel[k];
-                du[1 + k] = ma - mb;
-            }
-            du[D + 1] = qi.u[D + 1] - qn.u[D + 1];
+            for (int s = 0; s < NS; ++s) du[s] = qi.u[s] - qn.u[s];
             viscous_jump64<D>(qi, du, nh, pc, ja);
             viscous_jump64<D>(qn, du, nh, pc, jb);
             double pen = a.penalty;
