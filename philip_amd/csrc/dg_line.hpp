@@ -531,19 +531,21 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
         node_fill<double, D>(qn, fc);
     }
-    // the jump of the energy itself (Lax-Friedrichs, SIPG), and of the momentum itself (SIPG): rebuilt
-    // from the cache, they would leave a jump of their own rounding
+    // the jump of the energy itself (Lax-Friedrichs, SIPG), and of the momentum itself (SIPG, and with
+    // the viscous terms or on a curvilinear grid all but the two-point fluxes without Lax-Friedrichs
+    // dissipation): rebuilt from the cache, they would leave a jump of their own rounding
+    constexpr bool MOM = FORM == FORM_CONS || V || CV;
     if (energy_in_sr(pc.conv_flux)) {
         qi.u[D + 1] = qi.sr;
         if (nbl >= 0) qn.u[D + 1] = qn.sr;
     }
-    if (V && pc.diss_flux == 0) {
+    if ((V && pc.diss_flux == 0) || (MOM && FORM != FORM_CONS && pc.conv_flux != 3 && pc.conv_flux != 5)) {
         for (int s = 1; s < NS; ++s) qi.u[s] = a.u[((long)e * NS + s) * NP + fi];
         if (nbl >= 0)
             for (int s = 1; s < NS; ++s) qn.u[s] = a.u[((long)nb * NS + s) * NP + fj];
     }
     double fs[NS];
-    num_flux64<D, K, CV, FORM == FORM_GEN, FORM == FORM_CONS>(qi, qn, sgn, nh, own, fc, pc, fs);
+    num_flux64<D, K, CV, FORM == FORM_GEN, MOM>(qi, qn, sgn, nh, own, fc, pc, fs);
     const double iwb = ops.inv_wb;
     const double w = CV ? iwb * area : iwb;
     for (int s = 0; s < NS; ++s) {
