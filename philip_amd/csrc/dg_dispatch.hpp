@@ -25,20 +25,18 @@ inline int check_launch(dgx_ctx *c, const char *what)
     return DGX_OK;
 }
 
-// The small meshes' block of the line kernel, if the mesh is one; tells whether it was launched.
-// A mesh of at most a block per compute unit is bound by the length of one block's chain, not by
-// throughput.  Right-hand side, default -> small, at 0.4 blocks per unit: FP64 2D p=2 7.6 -> 5.6
-// us, p=4 9.6 -> 5.9, p=6 11.1 -> 7.9; 3D p=1 10.6 -> 6.0, p=3 10.0 -> 6.1, p=5 12.2 -> 8.2; mixed 3D
-// p=3 10.3 -> 6.2.  At one block per unit they meet (3D p=2 10.0 and 10.1, p=4 11.7 and 12.0); with
-// 1.5 the small blocks are slower.  FP64 p=6 in 3D would spill.
+// The small meshes' block of the line kernel, if the mesh is one (takes_small_block); tells whether it
+// was launched.
 template <int D, int N, typename T, int FORM>
 bool line_small_dn(dgx_ctx *c, const StageArgs &a)
 {
-    if constexpr (FORM != FORM_GEN && !(D == 3 && N == 7 && std::is_same<T, double>::value)) {
+    constexpr bool FP64 = std::is_same<T, double>::value;
+    if constexpr (has_small_block(D, N, FP64, FORM)) {
         using LS = LineGeoSmall<D, N, T>;
-        constexpr int EPB = LineGeoS<D, N, T>::EPB;
-        if (c->has_boundary || (c->ncells + EPB - 1) / EPB > c->n_cu) return false;
-        hipLaunchKernelGGL((line_kernel_small<D, N, T, FORM>), dim3((c->ncells + LS::EPB - 1) / LS::EPB),
+        const int blocks = (c->ncells + block_elements(D, N) - 1) / block_elements(D, N);
+        const int small = (c->ncells + LS::EPB - 1) / LS::EPB;
+        if (c->has_boundary || !takes_small_block(D, N, FP64, FORM, blocks, small, c->n_cu)) return false;
+        hipLaunchKernelGGL((line_kernel_small<D, N, T, FORM>), dim3(small),
                            dim3(LS::BLOCK), 0, c->stream, a, c->ops, c->pc);
         return true;
     }

@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "dg_physics.hpp"
+#include "dg_rules.hpp"
 
 namespace dgx {
 
@@ -274,17 +275,12 @@ __device__ __forceinline__ void ec_flux64(const NodeC<double, D> &a, const NodeC
     }
 }
 
-// Volume form of an FP64 line kernel: Chandrashekar / Ranocha split form, the split form with one of
-// the other two-point fluxes (a kernel of its own: the generic evaluation sets the register count of
-// a kernel that holds both -- p=3: 153 VGPRs, the curved kernel 246), the conservative form.
-enum LineForm { FORM_EC = 0, FORM_GEN = 1, FORM_CONS = 2 };
-
 // What a form keeps in two fields of a node's FP64 cache (rho, v, p, beta, H, c, sqrt(rho)): the
 // conservative form the momentum in the velocity's place and 1/rho in beta's, so that the mass flux is
 // the momentum itself, as it is in a trace; Kennedy-Gruber and Ismail-Roe, which have no beta, E there.
 // Lax-Friedrichs dissipation, which does not read sqrt(rho), has E in that field in every form
 // (energy_in_sr): read from memory by the face items instead, E was a round trip in the middle of the
-// line phase (conservative rhs 3D p=3 small mesh 5.9 -> 6.4 us, default block p=5 7.9 -> 9.9 us).
+// line phase (conservative rhs in small blocks, 3D p=1 20^3 12.3 -> 10.1 us, p=2 13^3 11.0 -> 8.9 us).
 __device__ __forceinline__ bool energy_in_sr(int conv_flux) { return conv_flux == 0 || conv_flux == 4; }
 template <int D, int FORM>
 __device__ __forceinline__ void node_to_cache64(const FastConst<double> &fc, NodeC<double, D> &n)

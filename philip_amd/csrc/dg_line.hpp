@@ -1090,12 +1090,7 @@ template <int D, int N, typename T> using LineGeoS = LineGeo<D, N, T, line_es_si
 
 // Small meshes: fewer elements per block, so that a mesh that cannot fill the chip spreads over more
 // of it, and LINE_WAVES threads, so that a thread's chain is one item long instead of two or three.
-// Elements per block: what fills half a wave per (direction, part) of line items.
-template <int D, int N> constexpr int line_es_small()
-{
-    return 64 + (D == 2 ? (N == 2 ? 16 : N == 3 ? 10 : N == 4 ? 8 : N == 5 ? 6 : N == 6 ? 5 : 4)
-                        : (N == 2 ? 8 : N == 3 ? 3 : N == 4 ? 2 : 1));
-}
+template <int D, int N> constexpr int line_es_small() { return 64 + small_elements(D, N); }
 template <int D, int N, typename T> using LineGeoSmall = LineGeo<D, N, T, line_es_small<D, N>(), false, LINE_WAVES>;
 template <int D, int N, typename T, int FORM>
 __global__ void __launch_bounds__((LineGeoSmall<D, N, T>::BLOCK))

@@ -5,6 +5,50 @@
 
 namespace dgx {
 
+// Volume form of an FP64 line kernel: Chandrashekar / Ranocha split form, the split form with one of
+// the other two-point fluxes (a kernel of its own: the generic evaluation sets the register count of
+// a kernel that holds both -- p=3: 153 VGPRs, the curved kernel 246), the conservative form.
+enum LineForm { FORM_EC = 0, FORM_GEN = 1, FORM_CONS = 2 };
+
+// Elements of a 256-node block, and of a small meshes' block: what fills half a wave per (direction,
+// part) of line items.
+constexpr int block_elements(int dim, int n)
+{
+    const int np = dim == 3 ? n * n * n : n * n;
+    return np >= 256 ? 1 : 256 / np;
+}
+constexpr int small_elements(int dim, int n)
+{
+    return dim == 2 ? (n == 2 ? 16 : n == 3 ? 10 : n == 4 ? 8 : n == 5 ? 6 : n == 6 ? 5 : 4)
+                    : (n == 2 ? 8 : n == 3 ? 3 : n == 4 ? 2 : 1);
+}
+
+// Whether the line kernel of a form has the small meshes' block (the mixed kernels hold every two-point
+// flux in FORM_EC).  FP64 3D p=6 would spill; at 2D p=3 the conservative form and the generic fluxes
+// gain nothing (right-hand side, other kernel -> small: 4.5 -> 4.7 us; Ismail-Roe 13.3 -> 14.5).
+constexpr bool has_small_block(int dim, int n, bool fp64, int form)
+{
+    if (!fp64) return form == FORM_EC;
+    if (dim == 3 && n == 7) return false;
+    return form == FORM_EC || !(dim == 2 && n == 4);
+}
+
+// Whether a mesh, or the solves of a batched launch, of `blocks` 256-node blocks takes the small ones
+// (`small` of them).  With at most a block per compute unit a launch is bound by the length of one
+// block's chain, not by throughput.  Right-hand side, default -> small: FP64 at 0.5 blocks per unit 2D
+// p=2 7.5 -> 5.6 us, p=4 8.6 -> 5.9, p=6 10.7 -> 7.3; 3D p=1 9.4 -> 6.1, p=3 9.1 -> 6.6, p=5 12.6 -> 8.2;
+// Kennedy-Gruber 3D p=3 9.8 -> 6.9, 2D p=5 14.4 -> 7.5; at one block 2D p=3 7.1 -> 5.9, 3D p=2 10.1 and
+// 10.2, p=4 11.7 and 12.3.  Mixed 3D, whose default block has twice the elements at p=3, p=4, p=6: 1.0
+// blocks p=3 10.1 -> 6.5, p=4 13.0 -> 8.0, 1.7 blocks p=3 10.3 -> 13.9, 1.3 blocks p=6 17.7 -> 23.2.
+// Conservative form (phase kernel -> small) in 3D: as soon as a unit has more than two small blocks it
+// loses, p=2 444 blocks 9.0 -> 8.6, 576 blocks 9.0 -> 11.7, p=1 512 blocks 8.8 -> 7.9, 729 blocks 9.0 ->
+// 10.5; in 2D it does not, p=1 702 blocks 6.4 -> 5.3, p=2 689 blocks 6.5 -> 5.9.
+constexpr bool takes_small_block(int dim, int n, bool fp64, int form, int blocks, int small, int n_cu)
+{
+    if (!has_small_block(dim, n, fp64, form) || blocks > n_cu) return false;
+    return form != FORM_CONS || dim == 2 || small <= 2 * n_cu;
+}
+
 // Low-storage RK: whether the next stage's state is stored to stay in the caches for that stage's
 // read, or streamed like the other registers (stage_epilogue).  mb: size of the state in 10^6 bytes;
 // line: a line kernel, else stage2_kernel.  Step, streamed -> cached:

@@ -16,6 +16,11 @@ int main()
             double mb;
             std::cin >> line >> curved >> mb;
             std::cout << store_stays_cached(dim, n, line, curved, mb) << "\n";
+        } else if (rule == "small") {  // of a mesh of `cells` on 256 compute units
+            int fp64, form, cells;
+            std::cin >> fp64 >> form >> cells;
+            const int b = block_elements(dim, n), s = small_elements(dim, n);
+            std::cout << takes_small_block(dim, n, fp64, form, (cells + b - 1) / b, (cells + s - 1) / s, 256) << "\n";
         } else {
             return 1;
         }

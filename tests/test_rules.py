@@ -37,6 +37,21 @@ def test_store_policy(rules, dim, p, line, curved, mb, cached):
     assert rules("store", dim, p + 1, line, curved, mb) == cached
 
 
+EC, GEN, CONS = 0, 1, 2
+# dim, p, FP64, form, cells a side; faster in small blocks
+SMALL = [(3, 3, True, EC, 10, True), (3, 3, True, EC, 11, False), (2, 5, True, EC, 41, True), (3, 6, True, EC, 2, False),
+         (3, 3, False, EC, 10, True), (3, 3, False, EC, 12, False), (3, 4, False, EC, 8, True), (3, 4, False, EC, 9, False),
+         (3, 6, False, EC, 6, True), (3, 6, False, EC, 7, False), (2, 5, True, GEN, 29, True), (2, 3, True, GEN, 27, False),
+         (3, 1, True, CONS, 16, True), (3, 1, True, CONS, 18, False), (3, 2, True, CONS, 11, True),
+         (3, 2, True, CONS, 12, False), (2, 3, True, CONS, 14, False), (2, 4, True, CONS, 50, True),
+         (2, 1, True, CONS, 106, True)]
+
+
+@pytest.mark.parametrize("dim,p,fp64,form,n,small", SMALL)
+def test_small_meshes_block(rules, dim, p, fp64, form, n, small):
+    assert rules("small", dim, p + 1, fp64, form, n ** dim) == small
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
 def test_both_store_policies_are_in_the_code(tmp_path):
     """The state's four stores once streamed and once not, beside S2's four streamed ones."""
