@@ -62,11 +62,6 @@ void line_dn(dgx_ctx *c, const StageArgs &a)
     else go(std::false_type{});
 }
 
-// FP64 conservative form on the box: the line kernel in 3D up to p=5 (rhs of 28^3 p=3 67 -> 54 us, 16^3
-// p=5 51 -> 42 us); in 2D (300^2 p=4 62 against 67 us) and at p=6 (14^3 71 against 77 us) stage2_kernel,
-// small meshes apart.
-template <int D, int N> constexpr bool line_conservative() { return D == 3 && N <= 6; }
-
 // Stage kernel of a context.  FP64: the line kernel, but for walls with the viscous terms, boundary
 // faces on a curvilinear grid, and Kennedy-Gruber or Ismail-Roe fluxes with the viscous terms or on a
 // curvilinear grid, which are stage2_kernel's.  Mixed: the line kernel for the periodic split form and
@@ -81,11 +76,11 @@ void stage2_dn(dgx_ctx *c, StageArgs a, dim3 grid, dim3 block)
     a.s1_cached = store_stays_cached(D, N, true, curv, mb);
     if (!nsv && !curv) {
         if constexpr (FP64) {
-            if constexpr (line_conservative<D, N>()) {
-                if (!split) return line_dn<D, N, T, FORM_CONS>(c, a);
-            } else {
-                if (!split && line_small_dn<D, N, T, FORM_CONS>(c, a)) return;
-            }
+            if (!split && line_small_dn<D, N, T, FORM_CONS>(c, a)) return;
+            if constexpr (has_conservative_line(D, N))
+                if (!split && takes_conservative_line(D, N, bnd, a.mode == MODE_LSRK || a.mode == MODE_BUTCHER,
+                                                      (int)grid.x, c->n_cu))
+                    return line_dn<D, N, T, FORM_CONS>(c, a);
             if (split && c->pc.two_point < 2) return line_dn<D, N, T, FORM_GEN>(c, a);
         }
         if (split) return line_dn<D, N, T, FORM_EC>(c, a);
@@ -154,10 +149,8 @@ void stage2_dn(dgx_ctx *c, StageArgs a, dim3 grid, dim3 block)
         else go2(no, no, yes, yes);
         return;
     }
-    if constexpr (!FP64 || !line_conservative<D, N>()) {  // conservative Euler on the box
-        if (bnd) go2(no, no, yes, no);
-        else go2(no, no, no, no);
-    }
+    if (bnd) go2(no, no, yes, no);  // conservative Euler on the box
+    else go2(no, no, no, no);
 }
 
 template <int D, int N>

@@ -49,6 +49,26 @@ constexpr bool takes_small_block(int dim, int n, bool fp64, int form, int blocks
     return form != FORM_CONS || dim == 2 || small <= 2 * n_cu;
 }
 
+// FP64 conservative form on the box, the small meshes' block apart: whether `blocks` 256-node blocks go
+// to the line kernel, else to stage2_kernel.  The line kernel, in 3D up to p=5, needs half the time at
+// many blocks per compute unit and more than the phase kernel at few; in a stage of a step, whose
+// registers it loads ahead, it wins from one block on (p=3 12^3, 1.7 blocks: 5 stages 71 -> 62 us, p=5
+// 7^3, 1.3 blocks: 69 -> 64).  Right-hand side, stage2_kernel ->
+// line kernel, Roe and Lax-Friedrichs: p=3 0.7 blocks per unit 7.1 -> 9.2 and 5.9 -> 8.4 us, 1.7 blocks
+// 9.8 -> 10.3 and 7.7 -> 9.4, 3.3 blocks 17.8 -> 14.4 and 13.9 -> 12.4, 24 blocks 89 -> 64 and 72 -> 56; p=5
+// 2.0 blocks 10.2 -> 11.0 and 7.9 -> 9.9, 3.9 blocks 19.4 -> 14.8 and 15.6 -> 13.2; p=2 at 1.5 blocks
+// already 12.9 -> 10.9 and 9.3 -> 9.5.  With boundary faces the line kernel is the faster one
+// throughout (p=3 0.3 blocks 9.6 and 9.6, 1.7 blocks 13.4 -> 10.9) but for p=1 (0.7 blocks 11.5 -> 12.3,
+// 1.5 blocks 16.2 -> 14.4).  Elsewhere stage2_kernel is: 2D p=4 300^2 62 against 67 us, 3D p=6 14^3 71
+// against 77 us.
+constexpr bool has_conservative_line(int dim, int n) { return dim == 3 && n <= 6; }
+constexpr bool takes_conservative_line(int dim, int n, bool boundary, bool stage, int blocks, int n_cu)
+{
+    if (!has_conservative_line(dim, n)) return false;
+    if (boundary) return n != 2 || blocks > n_cu;
+    return blocks > (n == 3 || stage ? 1 : 2) * n_cu;
+}
+
 // Low-storage RK: whether the next stage's state is stored to stay in the caches for that stage's
 // read, or streamed like the other registers (stage_epilogue).  mb: size of the state in 10^6 bytes;
 // line: a line kernel, else stage2_kernel.  Step, streamed -> cached:

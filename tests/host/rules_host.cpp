@@ -21,6 +21,11 @@ int main()
             std::cin >> fp64 >> form >> cells;
             const int b = block_elements(dim, n), s = small_elements(dim, n);
             std::cout << takes_small_block(dim, n, fp64, form, (cells + b - 1) / b, (cells + s - 1) / s, 256) << "\n";
+        } else if (rule == "conservative") {
+            int boundary, stage, cells;
+            std::cin >> boundary >> stage >> cells;
+            const int b = block_elements(dim, n);
+            std::cout << takes_conservative_line(dim, n, boundary, stage, (cells + b - 1) / b, 256) << "\n";
         } else {
             return 1;
         }

@@ -52,6 +52,20 @@ def test_small_meshes_block(rules, dim, p, fp64, form, n, small):
     assert rules("small", dim, p + 1, fp64, form, n ** dim) == small
 
 
+# dim, p, boundary faces, stage of a step, cells a side; faster in the line kernel
+CONSERVATIVE = [(3, 3, False, False, 12, False), (3, 3, False, True, 12, True), (3, 3, False, False, 15, True),
+                (3, 5, False, False, 8, False), (3, 5, False, True, 7, True), (3, 5, False, False, 10, True),
+                (3, 2, False, False, 13, False), (3, 2, False, False, 15, True), (3, 1, False, False, 23, False),
+                (3, 1, False, True, 23, True), (3, 1, False, True, 20, False), (3, 1, False, False, 30, True),
+                (3, 6, False, False, 14, False), (2, 4, False, True, 300, False), (3, 3, True, False, 7, True),
+                (3, 1, True, False, 18, False), (3, 1, True, False, 23, True)]
+
+
+@pytest.mark.parametrize("dim,p,boundary,stage,n,line", CONSERVATIVE)
+def test_conservative_line_kernel(rules, dim, p, boundary, stage, n, line):
+    assert rules("conservative", dim, p + 1, boundary, stage, n ** dim) == line
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
 def test_both_store_policies_are_in_the_code(tmp_path):
     """The state's four stores once streamed and once not, beside S2's four streamed ones."""
