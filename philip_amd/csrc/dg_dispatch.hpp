@@ -73,7 +73,7 @@ void stage2_dn(dgx_ctx *c, StageArgs a, dim3 grid, dim3 block)
     const bool split = c->P.use_split_form != 0, bnd = c->has_boundary, curv = c->curv;
     const bool nsv = D == 3 && c->P.pde == DGX_NAVIER_STOKES;
     const double mb = 1e-6 * sizeof(double) * c->ncells * Geo<D, N>::NS * Geo<D, N>::NP;
-    a.s1_cached = store_stays_cached(D, N, true, curv, mb);
+    a.s1_cached = store_stays_cached(D, N, FP64, true, curv, mb);
     if (!nsv && !curv) {
         if constexpr (FP64) {
             if (!split && line_small_dn<D, N, T, FORM_CONS>(c, a)) return;
@@ -118,7 +118,7 @@ void stage2_dn(dgx_ctx *c, StageArgs a, dim3 grid, dim3 block)
             return;
         }
     }
-    a.s1_cached = store_stays_cached(D, N, false, curv, mb);
+    a.s1_cached = store_stays_cached(D, N, FP64, false, curv, mb);
     auto go2 = [&](auto sc, auto vc, auto bc, auto cc) {
         hipLaunchKernelGGL((stage2_kernel<D, N, decltype(sc)::value, decltype(vc)::value, T, decltype(bc)::value,
                                           decltype(cc)::value>),

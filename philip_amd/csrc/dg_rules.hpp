@@ -79,16 +79,16 @@ constexpr bool takes_conservative_line(int dim, int n, bool boundary, bool stage
 //   box, line kernels: FP64 3D p=3 62 MB 510 -> 483, 119 MB 934 -> 896, 250 MB and above the same
 //     within 1 %; mixed 119 MB 753 -> 714; 2D p=1 96 MB 1390 -> 999 and 320 MB 1.37 times
 //   stage2_kernel: the state is not the largest part of its traffic.  Conservative, 3D, FP64 p=6 18 MB
-//     324 -> 315, 56 MB 857 -> 813, 127 MB 1949 -> 1973; mixed p=3 20 MB 148 -> 155, p=2 84 MB 1.02
+//     324 -> 315, 24 MB 386 -> 367, 56 MB 857 -> 813, 127 MB 1949 -> 1973; mixed p=3 20 MB 148 -> 155, p=2 84 MB 1.02
 //     times, 119 MB 867 -> 883; 2D p=1 and p=2 always (96 MB 996 -> 840, 864 -> 737), p=3 48 MB 257 ->
 //     261, p=4 48 MB 316 -> 296, p=5 134 MB 0.96 times
 //   curvilinear, 3D from p=3: the metric terms need the cache.  FP64 p=3 62 MB 628 -> 584, 84 MB 0.95
 //     times, 119 MB 1192 -> 1201, p=4 122 MB 1772 -> 1781; p=1 59 MB 781 -> 710, 170 MB and above 1.02
-constexpr bool store_stays_cached(int dim, int n, bool line, bool curved, double mb)
+constexpr bool store_stays_cached(int dim, int n, bool fp64, bool line, bool curved, double mb)
 {
     if (mb < (dim == 2 && n <= 3 ? 6.0 : 12.0)) return false;
     if (curved && dim == 3 && n >= 4) return mb <= 64.0;
-    if (!line && dim == 3) return mb >= 40.0 && mb <= 100.0;
+    if (!line && dim == 3) return mb >= (fp64 ? 12.0 : 40.0) && mb <= 100.0;
     if (!line && n >= 4) return mb <= 100.0;
     return true;
 }

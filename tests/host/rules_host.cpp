@@ -12,10 +12,10 @@ int main()
         int dim, n;
         std::cin >> dim >> n;
         if (rule == "store") {
-            int line, curved;
+            int fp64, line, curved;
             double mb;
-            std::cin >> line >> curved >> mb;
-            std::cout << store_stays_cached(dim, n, line, curved, mb) << "\n";
+            std::cin >> fp64 >> line >> curved >> mb;
+            std::cout << store_stays_cached(dim, n, fp64, line, curved, mb) << "\n";
         } else if (rule == "small") {  // of a mesh of `cells` on 256 compute units
             int fp64, form, cells;
             std::cin >> fp64 >> form >> cells;

@@ -24,17 +24,18 @@ def rules(tmp_path_factory):
     return ask
 
 
-# dim, p, line kernel, curved, state in MB; faster cached
-STORE = [(3, 3, True, False, 8.6, False), (3, 3, True, False, 84, True), (3, 3, True, False, 119, True),
-         (2, 1, True, False, 3.2, False), (2, 2, False, False, 7.1, True), (2, 1, True, False, 320, True), (3, 3, False, False, 20, False),
-         (3, 2, False, False, 84, True), (3, 6, False, False, 127, False), (2, 3, False, False, 134, False),
-         (2, 1, False, False, 134, True), (3, 3, True, True, 62, True), (3, 3, True, True, 84, False),
-         (3, 1, True, True, 170, True), (3, 4, False, True, 122, False)]
+# dim, p, FP64, line kernel, curved, state in MB; faster cached
+STORE = [(3, 3, True, True, False, 8.6, False), (3, 3, True, True, False, 84, True), (3, 3, False, True, False, 119, True),
+         (2, 1, False, True, False, 3.2, False), (2, 2, False, False, False, 7.1, True), (2, 1, True, True, False, 320, True),
+         (3, 3, False, False, False, 20, False), (3, 6, True, False, False, 24, True), (3, 2, False, False, False, 84, True),
+         (3, 6, True, False, False, 127, False), (2, 3, False, False, False, 134, False), (2, 1, False, False, False, 134, True),
+         (3, 3, True, True, True, 62, True), (3, 3, True, True, True, 84, False), (3, 1, True, True, True, 170, True),
+         (3, 4, False, False, True, 122, False)]
 
 
-@pytest.mark.parametrize("dim,p,line,curved,mb,cached", STORE)
-def test_store_policy(rules, dim, p, line, curved, mb, cached):
-    assert rules("store", dim, p + 1, line, curved, mb) == cached
+@pytest.mark.parametrize("dim,p,fp64,line,curved,mb,cached", STORE)
+def test_store_policy(rules, dim, p, fp64, line, curved, mb, cached):
+    assert rules("store", dim, p + 1, fp64, line, curved, mb) == cached
 
 
 EC, GEN, CONS = 0, 1, 2
