@@ -997,12 +997,12 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
         }
     }
     __syncthreads();  // node cache and traces consumed; their storage now takes the partials
-    // FP64: the registers of the epilogue are read from here on; mixed: those of a Butcher stage (S2
-    // and S3 were loaded in phase A; 2D p=3 512^2 RK4 stage 157 -> 128 us, Navier-Stokes p=5 16^3 147 ->
-    // 129 us with the lifted gradient)
+    // FP64: the registers of the epilogue are read from here on; mixed: those of a Butcher stage where
+    // that is faster (S2 and S3 were loaded in phase A)
     constexpr bool LATE_PF = FAST || line_late_prefetch_d<D, N>();
     const bool late_pf = LATE_PF && active &&
-                         ((!EARLY && a.mode == MODE_LSRK && !a.lsrk_first) || a.mode == MODE_BUTCHER);
+                         ((!EARLY && a.mode == MODE_LSRK && !a.lsrk_first) ||
+                          (butcher_prefetch(D, N, !FAST) && a.mode == MODE_BUTCHER));
     // FP64 at N >= 4: the stage state is read again here for the epilogue (an L2 hit: the block
     // read it in phase A) instead of being held in registers through the line phase (TGV 32^3
     // p=3: 177 -> 170 us per stage, 64 -> 16 B/lane of spills; p=4 24^3 294 -> 244 us; at p=2

@@ -69,6 +69,12 @@ constexpr bool takes_conservative_line(int dim, int n, bool boundary, bool stage
     return blocks > (n == 3 || stage ? 1 : 2) * n_cu;
 }
 
+// Whether a line kernel loads a Butcher stage's registers before the line sums go to LDS rather than in
+// the epilogue.  Mixed RK4 step, epilogue -> before: 2D p=3 96 MB 454 -> 377 us, 3D p=3 119 MB 769 -> 626,
+// Navier-Stokes p=5 16^3 stage with the lifted gradient 147 -> 129; but 2D p=1 48 MB 212 -> 257, p=2 216 ->
+// 235 (96 MB 540 -> 496).
+constexpr bool butcher_prefetch(int dim, int n, bool fp64) { return fp64 || dim == 3 || n >= 4; }
+
 // Low-storage RK: whether the next stage's state is stored to stay in the caches for that stage's
 // read, or streamed like the other registers (stage_epilogue).  mb: size of the state in 10^6 bytes;
 // line: a line kernel, else stage2_kernel.  Step, streamed -> cached:

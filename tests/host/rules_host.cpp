@@ -26,6 +26,10 @@ int main()
             std::cin >> boundary >> stage >> cells;
             const int b = block_elements(dim, n);
             std::cout << takes_conservative_line(dim, n, boundary, stage, (cells + b - 1) / b, 256) << "\n";
+        } else if (rule == "prefetch") {
+            int fp64;
+            std::cin >> fp64;
+            std::cout << butcher_prefetch(dim, n, fp64) << "\n";
         } else {
             return 1;
         }

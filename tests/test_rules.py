@@ -67,6 +67,12 @@ def test_conservative_line_kernel(rules, dim, p, boundary, stage, n, line):
     assert rules("conservative", dim, p + 1, boundary, stage, n ** dim) == line
 
 
+@pytest.mark.parametrize("dim,p,fp64,early", [(2, 1, False, False), (2, 2, False, False), (2, 3, False, True),
+                                              (3, 1, False, True), (2, 1, True, True)])
+def test_butcher_prefetch(rules, dim, p, fp64, early):
+    assert rules("prefetch", dim, p + 1, fp64) == early
+
+
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="no hipcc")
 def test_both_store_policies_are_in_the_code(tmp_path):
     """The state's four stores once streamed and once not, beside S2's four streamed ones."""
