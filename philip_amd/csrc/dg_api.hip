@@ -1318,6 +1318,22 @@ static bool batch_line_eligible(const dgx_ctx *c)
     return c->P.use_split_form && c->P.pde == DGX_EULER && !c->has_boundary && !c->curv;
 }
 
+// The small meshes' tile if solves that fill a batched launch together take it (takes_small_block, the
+// rule of a single solve), else -1.  It is chosen by this rule alone and never timed: its merit hangs
+// on the work of a launch, and a tile once timed serves every later group of its shape.
+template <typename Cells> static int small_tile(const dgx_ctx *c, const Cells &ncells)
+{
+    const int eb = block_elements(c->dim, c->n), es = small_elements(c->dim, c->n);
+    int blocks = 0, small = 0;
+    for (int k : ncells) {
+        blocks += (k + eb - 1) / eb;
+        small += (k + es - 1) / es;
+    }
+    const bool fp64 = c->P.precision == DGX_FP64;
+    const int form = batch_generic(c) ? FORM_GEN : FORM_EC;
+    return takes_small_block(c->dim, c->n, fp64, form, blocks, small, c->n_cu) ? batch_tile_small(c->dim) : -1;
+}
+
 // block table of a group for `epb` elements per block: (slot, first element) per element group
 static int group_table(dgx_batch *b, const BatchGroup &g, int epb, BatchBlock **out, int *nblocks)
 {
@@ -1347,11 +1363,15 @@ static int batch_blocks(dgx_batch *b, BatchGroup &g, int tile)
     return DGX_OK;
 }
 
-// Times every candidate tile (batch_tile) on the group's first RK stage (median of seven
-// launches after a warm-up) and keeps the fastest.
+// Times every candidate tile (batch_tile but for the small meshes', see small_tile) on the group's
+// first RK stage (median of seven launches after a warm-up) and keeps the fastest.
 static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
 {
     if (b->forced_tile >= 0 && batch_blocks(b, g, b->forced_tile) == DGX_OK) return DGX_OK;
+    std::vector<int> ncells;
+    for (int i : g.inst) ncells.push_back(b->inst[i]->ncells);
+    const int st = small_tile(b->inst[g.inst[0]], ncells);
+    if (st >= 0) return batch_blocks(b, g, st);
     const long key = (((long)g.dim * 16 + g.n) * 4 + g.precision) * 2 + g.generic;
     for (auto &kv : g_variant_cache)
         if (kv.first == key) return batch_blocks(b, g, kv.second);
@@ -1365,7 +1385,7 @@ static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
     // drift of the clock or of the other groups' caches during tuning biases no candidate
     std::vector<int> cand, table;                 // candidate tiles, index of their block table
     std::vector<std::pair<int, std::pair<BatchBlock *, int>>> tables;  // epb -> (table, blocks)
-    for (int tile = 0; tile < batch_tile_count(g.dim); ++tile) {
+    for (int tile = 0; tile < batch_tile_small(g.dim); ++tile) {
         int epb = 0;
         if (launch_line_batch(g.dim, g.n, g.precision, g.generic, tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &epb))
             continue;  // tile does not fit this shape
@@ -1818,17 +1838,13 @@ static int server_advance(dgx_server *s)
         grouped[k] = true;
     }
     for (G &g : groups) {
-        // a group that does not fill the chip in the default tile takes the small meshes'
-        int blocks = 0;
-        for (int k : g.members) blocks += (s->active[k].c->ncells + g.epb - 1) / g.epb;
-        if (g.tile == 0 && blocks <= s->active[g.members[0]].c->n_cu) {
-            int epb = 0;
-            if (launch_line_batch(g.dim, g.n, g.precision, g.generic, batch_tile_small(g.dim), nullptr, 0, nullptr,
-                                  nullptr, Ops1D{}, nullptr, &epb) == DGX_OK) {
-                g.tile = batch_tile_small(g.dim);
-                g.epb = epb;
-            }
-        }
+        // a group that does not fill the chip takes the small meshes' tile, whatever tile was timed
+        std::vector<int> ncells;
+        for (int k : g.members) ncells.push_back(s->active[k].c->ncells);
+        const int st = small_tile(s->active[g.members[0]].c, ncells);
+        if (st < 0) continue;
+        g.tile = st;
+        launch_line_batch(g.dim, g.n, g.precision, g.generic, st, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &g.epb);
     }
     // pack the tables
     int64_t bytes = 0;

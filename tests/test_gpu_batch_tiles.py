@@ -40,3 +40,18 @@ def test_no_tile_for_a_block_that_single_solves_do_not_take():
     b = batch([params(3, 6, 3)] * 2, tile=2)
     assert b.tile(0)[2] != 768
     b.close()
+
+
+@pytest.mark.parametrize("precision", [P.FP64, P.MIXED])
+@pytest.mark.parametrize("first", ["tiny", "large"])
+def test_tile_follows_the_batch_and_not_what_ran_before(first, precision):
+    """A batch that leaves most of the chip idle takes the small meshes' tile, one that fills it a timed
+    tile, in either order and again."""
+    p = 1 if first == "tiny" else 4  # a shape of its own for each order
+    tiny, large = [params(2, p, 8, precision=precision)] * 2, [params(2, p, 128, precision=precision)] * 4
+    order = [tiny, large, tiny, large] if first == "tiny" else [large, tiny, large]
+    for cases in order:
+        b = batch(cases)
+        print(first, precision, len(cases), b.tile(0), flush=True)
+        assert (b.tile(0)[0] == SMALL_2D[p]) == (cases is tiny)
+        b.close()
