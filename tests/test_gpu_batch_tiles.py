@@ -55,3 +55,52 @@ def test_tile_follows_the_batch_and_not_what_ran_before(first, precision):
         print(first, precision, len(cases), b.tile(0), flush=True)
         assert (b.tile(0)[0] == SMALL_2D[p]) == (cases is tiny)
         b.close()
+
+
+@pytest.mark.parametrize("tp", [P.KG, P.IR])
+@pytest.mark.parametrize("dim,p,n", [(2, 2, 9), (2, 4, 7), (2, 5, 40), (3, 3, 4), (3, 5, 3)])
+def test_generic_fluxes_in_a_batch(dim, p, n, tp):
+    cases = [params(dim, p, n, t, prec) for t in (tp, P.CH) for prec in (P.FP64, P.MIXED)]
+    cases.append(params(dim, p, n + 1, tp, cf=P.TWO_POINT_LXF))
+    alone = []
+    for kw in cases:
+        d = P.DG(**kw)
+        start(d, dim)
+        d.allocate_ode_system("rk4")
+        d.step_in_time(d.constant_time_step(0.01), 2)
+        alone.append(d.solution())
+        d.close()
+    for tile in [-1] + list(range(13 if dim == 2 else 3)):
+        print(dim, p, n, tp, tile, flush=True)
+        b = batch(cases, tile, 2)
+        if tile == 0:
+            assert all(b.variant(i) == 1 for i in range(len(cases)))
+        assert all(b.variant(i) > 0 for i in range(len(cases)))
+        for d, u in zip(b.instances, alone):
+            assert np.array_equal(d.solution(), u)
+        b.close()
+
+
+def test_generic_fluxes_in_a_stream():
+    specs = []
+    for k, tp in enumerate([P.CH, P.KG, P.IR, P.KG, P.CH, P.IR]):
+        dim = 3 if k % 3 == 2 else 2
+        spec = dict(final_time=0.01 + 0.004 * k, cfl=0.02, wave_speed=2.0, ic=P.IC_TGV if dim == 3 else P.IC_VORTEX,
+                    vortex=(5.0, 0.5, 0.6))
+        specs.append((params(dim, 3, 4 if dim == 3 else 9, tp), spec))
+    s = P.Server(1 << 30, max_active=8)
+    ids = [s.submit(P.request(**spec, **kw)) for kw, spec in specs]
+    while True:
+        a, q, _ = s.step()
+        if not a and not q:
+            break
+    for i, (kw, spec) in zip(ids, specs):
+        d = P.DG(**kw)
+        if kw["dim"] == 2:
+            d.set_initial_condition_vortex(*spec["vortex"])
+        else:
+            d.set_initial_condition_tgv()
+        d.run("rk4", d.constant_time_step(spec["cfl"]) / spec["wave_speed"], spec["final_time"])
+        assert np.array_equal(s.result(i)[0], d.solution())
+        d.close()
+    s.close()
