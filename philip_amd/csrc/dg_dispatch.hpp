@@ -213,11 +213,8 @@ int line_batch_es(const BatchBlock *blocks, int nblocks, const StageArgs *args, 
                   const Ops1D &ops, hipStream_t st, int *epb, int *threads)
 {
     using LG = LineGeo<D, N, T, ES, false, XJ>;
-    constexpr bool SMALL = XJ == LINE_WAVES;
-    if constexpr (LG::SBUF * sizeof(T) > 160 * 1024 - 4096 || LG::BLOCK > 1024 ||
-                  (SMALL && !has_small_block(D, N, std::is_same<T, double>::value, GEN ? FORM_GEN : FORM_EC))) {
-        // would not fit the 160 KB of LDS or the 1024 threads of a block; no small meshes' block
-        return DGX_ERR_UNSUPPORTED;
+    if constexpr (LG::SBUF * sizeof(T) > 160 * 1024 - 4096 || LG::BLOCK > 1024) {
+        return DGX_ERR_UNSUPPORTED;  // would not fit the 160 KB of LDS or the 1024 threads of a block
     } else {
         if (epb) *epb = LG::EPB;
         if (threads) *threads = LG::BLOCK;

@@ -35,13 +35,6 @@ def batch(cases, tile=-1, steps=0):
     return b
 
 
-def test_no_tile_for_a_block_that_single_solves_do_not_take():
-    """FP64 3D p=6: the small meshes' block (768 threads) would spill."""
-    b = batch([params(3, 6, 3)] * 2, tile=2)
-    assert b.tile(0)[2] != 768
-    b.close()
-
-
 @pytest.mark.parametrize("precision", [P.FP64, P.MIXED])
 @pytest.mark.parametrize("first", ["tiny", "large"])
 def test_tile_follows_the_batch_and_not_what_ran_before(first, precision):
