@@ -1265,7 +1265,7 @@ struct BatchGroup {
     std::vector<StageArgs *> args;       // device, per stage: per slot
 };
 
-// batched tile chosen per (dim, n, precision) in this process
+// batched tile timed per shape and load (tile_key) in this process
 std::vector<std::pair<long, int>> g_variant_cache;
 
 } // namespace
@@ -1318,20 +1318,23 @@ static bool batch_line_eligible(const dgx_ctx *c)
     return c->P.use_split_form && c->P.pde == DGX_EULER && !c->has_boundary && !c->curv;
 }
 
-// The small meshes' tile if solves that fill a batched launch together take it (takes_small_block, the
-// rule of a single solve), else -1.  It is chosen by this rule alone and never timed: its merit hangs
-// on the work of a launch, and a tile once timed serves every later group of its shape.
-template <typename Cells> static int small_tile(const dgx_ctx *c, const Cells &ncells)
+// Load of a batched launch: 256-node blocks of its solves per compute unit, in powers of four; 0: at most
+// one.  There the small meshes' tile is taken without timing, as in a single solve (takes_small_block:
+// the longest chain of a block is all that counts).  Above it which tile is best hangs on the load as
+// well (the small meshes' one is the fastest at 2D p=3 with 5 blocks a unit, 100 against 120 us a step,
+// and the slowest at 3D p=3 mixed, 217 against 164), so a timed tile serves only its own class.
+template <typename Cells> static int batch_load(const dgx_ctx *c, const Cells &ncells)
 {
-    const int eb = block_elements(c->dim, c->n), es = small_elements(c->dim, c->n);
-    int blocks = 0, small = 0;
-    for (int k : ncells) {
-        blocks += (k + eb - 1) / eb;
-        small += (k + es - 1) / es;
-    }
-    const bool fp64 = c->P.precision == DGX_FP64;
-    const int form = batch_generic(c) ? FORM_GEN : FORM_EC;
-    return takes_small_block(c->dim, c->n, fp64, form, blocks, small, c->n_cu) ? batch_tile_small(c->dim) : -1;
+    const int eb = block_elements(c->dim, c->n);
+    long blocks = 0;
+    for (int k : ncells) blocks += (k + eb - 1) / eb;
+    int load = 0;
+    for (long most = c->n_cu; blocks > most; most *= 4) ++load;
+    return load;
+}
+static long tile_key(const dgx_ctx *c, int load)
+{
+    return ((((long)c->dim * 16 + c->n) * 4 + c->P.precision) * 2 + batch_generic(c)) * 32 + load;
 }
 
 // block table of a group for `epb` elements per block: (slot, first element) per element group
@@ -1363,16 +1366,16 @@ static int batch_blocks(dgx_batch *b, BatchGroup &g, int tile)
     return DGX_OK;
 }
 
-// Times every candidate tile (batch_tile but for the small meshes', see small_tile) on the group's
-// first RK stage (median of seven launches after a warm-up) and keeps the fastest.
+// Times every candidate tile (batch_tile) on the group's first RK stage (median of seven launches after
+// a warm-up) and keeps the fastest for groups of its shape and load.
 static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
 {
     if (b->forced_tile >= 0 && batch_blocks(b, g, b->forced_tile) == DGX_OK) return DGX_OK;
     std::vector<int> ncells;
     for (int i : g.inst) ncells.push_back(b->inst[i]->ncells);
-    const int st = small_tile(b->inst[g.inst[0]], ncells);
-    if (st >= 0) return batch_blocks(b, g, st);
-    const long key = (((long)g.dim * 16 + g.n) * 4 + g.precision) * 2 + g.generic;
+    const int load = batch_load(b->inst[g.inst[0]], ncells);
+    if (load == 0 && batch_blocks(b, g, batch_tile_small(g.dim)) == DGX_OK) return DGX_OK;
+    const long key = tile_key(b->inst[g.inst[0]], load);
     for (auto &kv : g_variant_cache)
         if (kv.first == key) return batch_blocks(b, g, kv.second);
     // the group's own first-stage launch: it reads u_n and writes only the accumulator and the
@@ -1385,7 +1388,7 @@ static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
     // drift of the clock or of the other groups' caches during tuning biases no candidate
     std::vector<int> cand, table;                 // candidate tiles, index of their block table
     std::vector<std::pair<int, std::pair<BatchBlock *, int>>> tables;  // epb -> (table, blocks)
-    for (int tile = 0; tile < batch_tile_small(g.dim); ++tile) {
+    for (int tile = 0; tile < batch_tile_count(g.dim); ++tile) {
         int epb = 0;
         if (launch_line_batch(g.dim, g.n, g.precision, g.generic, tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &epb))
             continue;  // tile does not fit this shape
@@ -1822,15 +1825,6 @@ static int server_advance(dgx_server *s)
             x.n = c->n;
             x.precision = c->P.precision;
             x.generic = batch_generic(c);
-            const long key = (((long)x.dim * 16 + x.n) * 4 + x.precision) * 2 + x.generic;
-            x.tile = 0;
-            for (auto &kv : g_variant_cache)
-                if (kv.first == key) x.tile = kv.second;
-            if (launch_line_batch(x.dim, x.n, x.precision, x.generic, x.tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
-                                  &x.epb) != DGX_OK) {
-                x.tile = 0;
-                launch_line_batch(x.dim, x.n, x.precision, x.generic, 0, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &x.epb);
-            }
             groups.push_back(x);
             g = &groups.back();
         }
@@ -1838,13 +1832,19 @@ static int server_advance(dgx_server *s)
         grouped[k] = true;
     }
     for (G &g : groups) {
-        // a group that does not fill the chip takes the small meshes' tile, whatever tile was timed
+        // the small meshes' tile or a tile that a batch of this shape and load has timed, else the default
+        const dgx_ctx *c = s->active[g.members[0]].c;
         std::vector<int> ncells;
         for (int k : g.members) ncells.push_back(s->active[k].c->ncells);
-        const int st = small_tile(s->active[g.members[0]].c, ncells);
-        if (st < 0) continue;
-        g.tile = st;
-        launch_line_batch(g.dim, g.n, g.precision, g.generic, st, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &g.epb);
+        const int load = batch_load(c, ncells);
+        g.tile = load == 0 ? batch_tile_small(g.dim) : 0;
+        for (auto &kv : g_variant_cache)
+            if (kv.first == tile_key(c, load)) g.tile = kv.second;
+        if (launch_line_batch(g.dim, g.n, g.precision, g.generic, g.tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
+                              &g.epb) != DGX_OK) {
+            g.tile = 0;
+            launch_line_batch(g.dim, g.n, g.precision, g.generic, 0, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr, &g.epb);
+        }
     }
     // pack the tables
     int64_t bytes = 0;
