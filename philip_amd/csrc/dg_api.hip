@@ -1318,22 +1318,25 @@ static bool batch_line_eligible(const dgx_ctx *c)
     return c->P.use_split_form && c->P.pde == DGX_EULER && !c->has_boundary && !c->curv;
 }
 
-// Load of a batched launch: 256-node blocks of its solves per compute unit, in powers of four; 0: at most
-// one.  There the small meshes' tile is taken without timing, as in a single solve (takes_small_block:
-// the longest chain of a block is all that counts).  Above it which tile is best hangs on the load as
-// well (the small meshes' one is the fastest at 2D p=3 with 5 blocks a unit, 100 against 120 us a step,
-// and the slowest at 3D p=3 mixed, 217 against 164), so a timed tile serves only its own class.
-template <typename Cells> static int batch_load(const dgx_ctx *c, const Cells &ncells)
+// 256-node blocks of the solves of a batched launch.
+template <typename Cells> static long batch_size(const dgx_ctx *c, const Cells &ncells)
 {
     const int eb = block_elements(c->dim, c->n);
     long blocks = 0;
     for (int k : ncells) blocks += (k + eb - 1) / eb;
+    return blocks;
+}
+static bool takes_small_tile(const dgx_ctx *c, long blocks)
+{
+    return batch_takes_small_tile(c->dim, c->n, c->P.precision == DGX_FP64, blocks, c->n_cu);
+}
+// A timed tile serves groups of its shape and load, the blocks per compute unit in powers of four: which
+// tile is best hangs on both (the small meshes' one is the fastest at 2D p=3 with 5 blocks a unit, 100
+// against 120 us a step, and the slowest at 3D p=3 mixed, 217 against 164).
+static long tile_key(const dgx_ctx *c, long blocks)
+{
     int load = 0;
     for (long most = c->n_cu; blocks > most; most *= 4) ++load;
-    return load;
-}
-static long tile_key(const dgx_ctx *c, int load)
-{
     return ((((long)c->dim * 16 + c->n) * 4 + c->P.precision) * 2 + batch_generic(c)) * 32 + load;
 }
 
@@ -1373,9 +1376,9 @@ static int batch_autotune(dgx_batch *b, BatchGroup &g, const Ops1D &ops)
     if (b->forced_tile >= 0 && batch_blocks(b, g, b->forced_tile) == DGX_OK) return DGX_OK;
     std::vector<int> ncells;
     for (int i : g.inst) ncells.push_back(b->inst[i]->ncells);
-    const int load = batch_load(b->inst[g.inst[0]], ncells);
-    if (load == 0 && batch_blocks(b, g, batch_tile_small(g.dim)) == DGX_OK) return DGX_OK;
-    const long key = tile_key(b->inst[g.inst[0]], load);
+    const dgx_ctx *c = b->inst[g.inst[0]];
+    const long blocks = batch_size(c, ncells), key = tile_key(c, blocks);
+    if (takes_small_tile(c, blocks) && batch_blocks(b, g, batch_tile_small(g.dim)) == DGX_OK) return DGX_OK;
     for (auto &kv : g_variant_cache)
         if (kv.first == key) return batch_blocks(b, g, kv.second);
     // the group's own first-stage launch: it reads u_n and writes only the accumulator and the
@@ -1836,10 +1839,11 @@ static int server_advance(dgx_server *s)
         const dgx_ctx *c = s->active[g.members[0]].c;
         std::vector<int> ncells;
         for (int k : g.members) ncells.push_back(s->active[k].c->ncells);
-        const int load = batch_load(c, ncells);
-        g.tile = load == 0 ? batch_tile_small(g.dim) : 0;
+        const long blocks = batch_size(c, ncells), key = tile_key(c, blocks);
+        const bool small = takes_small_tile(c, blocks);
+        g.tile = small ? batch_tile_small(g.dim) : 0;
         for (auto &kv : g_variant_cache)
-            if (kv.first == tile_key(c, load)) g.tile = kv.second;
+            if (!small && kv.first == key) g.tile = kv.second;
         if (launch_line_batch(g.dim, g.n, g.precision, g.generic, g.tile, nullptr, 0, nullptr, nullptr, Ops1D{}, nullptr,
                               &g.epb) != DGX_OK) {
             g.tile = 0;

@@ -1192,8 +1192,8 @@ line_kernel_batch_wb(const BatchBlock *__restrict__ blocks, const StageArgs *__r
 // occupancy) x threads per block (one per node, or one per line-phase item: XJ).  None changes
 // the arithmetic of an element (the line split LS is fixed per shape for that reason: it
 // reorders the pair sums), so every tile gives the single solve's bits.
-// The last tile is the small meshes' (line_es_small), taken without timing by groups of at most a block per
-// compute unit.
+// The last tile is the small meshes' (line_es_small), taken without timing by groups that do not fill the
+// chip (batch_takes_small_tile).
 struct BatchTile {
     int es, waves, xj;
 };

@@ -49,6 +49,17 @@ constexpr bool takes_small_block(int dim, int n, bool fp64, int form, int blocks
     return form != FORM_CONS || dim == 2 || small <= 2 * n_cu;
 }
 
+// Whether the solves of a batched launch, of `blocks` 256-node blocks in all, take the small meshes' tile
+// without timing.  RK4 step, default tile -> small, FP64: 2D p=4 0.5 blocks per unit 58 -> 46 us, 1.0 blocks
+// 69 -> 62; 3D p=3 57 -> 46 and 67 -> 62, p=6 84 -> 68 and 104 -> 88.  In 3D at p=2, and FP64 at p=1 and p=4,
+// the small blocks of one unit's worth of default ones no longer fit the chip at once: FP64 p=1 67 -> 48 and
+// 80 -> 88, p=2 64 -> 51 and 75 -> 83, p=4 69 -> 50 and 79 -> 91, mixed p=2 63 -> 48 and 74 -> 73.
+constexpr bool batch_takes_small_tile(int dim, int n, bool fp64, long blocks, int n_cu)
+{
+    const bool half = dim == 3 && (n == 3 || (fp64 && (n == 2 || n == 5)));
+    return blocks <= (half ? n_cu / 2 : n_cu);
+}
+
 // FP64 conservative form on the box, the small meshes' block apart: whether `blocks` 256-node blocks go
 // to the line kernel, else to stage2_kernel.  The line kernel, in 3D up to p=5, needs half the time at
 // many blocks per compute unit and more than the phase kernel at few; in a stage of a step, whose

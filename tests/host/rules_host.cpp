@@ -26,6 +26,11 @@ int main()
             std::cin >> boundary >> stage >> cells;
             const int b = block_elements(dim, n);
             std::cout << takes_conservative_line(dim, n, boundary, stage, (cells + b - 1) / b, 256) << "\n";
+        } else if (rule == "batch") {
+            int fp64;
+            long blocks;
+            std::cin >> fp64 >> blocks;
+            std::cout << batch_takes_small_tile(dim, n, fp64, blocks, 256) << "\n";
         } else if (rule == "prefetch") {
             int fp64;
             std::cin >> fp64;

@@ -67,6 +67,14 @@ def test_conservative_line_kernel(rules, dim, p, boundary, stage, n, line):
     assert rules("conservative", dim, p + 1, boundary, stage, n ** dim) == line
 
 
+@pytest.mark.parametrize("dim,p,fp64,blocks,small", [
+    (2, 4, True, 250, True), (2, 4, True, 350, False), (3, 3, True, 256, True), (3, 2, True, 125, True),
+    (3, 2, True, 182, False), (3, 4, True, 182, False), (3, 1, True, 253, False), (3, 1, False, 188, True),
+    (3, 2, False, 250, False), (3, 6, True, 256, True)])
+def test_batch_small_tile(rules, dim, p, fp64, blocks, small):
+    assert rules("batch", dim, p + 1, fp64, blocks) == small
+
+
 @pytest.mark.parametrize("dim,p,fp64,early", [(2, 1, False, False), (2, 2, False, False), (2, 3, False, True),
                                               (3, 1, False, True), (2, 1, True, True)])
 def test_butcher_prefetch(rules, dim, p, fp64, early):
