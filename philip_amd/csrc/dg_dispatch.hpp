@@ -64,7 +64,8 @@ void line_dn(dgx_ctx *c, const StageArgs &a)
 
 // Stage kernel of a context.  FP64: the line kernel, but for walls with the viscous terms, boundary
 // faces on a curvilinear grid, and Kennedy-Gruber or Ismail-Roe fluxes with the viscous terms or on a
-// curvilinear grid, which are stage2_kernel's.  Mixed: the line kernel for the periodic split form and
+// curvilinear grid, which are stage2_kernel's, as the conservative form on the box is in 2D, at p=6 and
+// on meshes of few blocks (takes_small_block, takes_conservative_line).  Mixed: the line kernel for the periodic split form and
 // for Euler boundary faces on the box, stage2_kernel for the rest.
 template <int D, int N, typename T>
 void stage2_dn(dgx_ctx *c, StageArgs a, dim3 grid, dim3 block)

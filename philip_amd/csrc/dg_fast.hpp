@@ -23,7 +23,7 @@
 // reciprocal serves both 1/(rho1+rho2) and 1/(b1+b2), 1/F_rho comes from its expansion and one
 // Newton step, and |avg v|^2 - avg |v|^2 / 2 is v1.v2 / 2.  Every sum over the two sides is written so that exchanging them and turning the
 // normal around gives the exact negative, so a face evaluated from either side needs no
-// selection of an owner.  They take a direction K or (CV) a normal / cofactor column nv.
+// selection of an owner (the Kennedy-Gruber and Ismail-Roe fluxes are ordered by it).  They take a direction K or (CV) a normal / cofactor column nv.
 #pragma once
 #include <type_traits>
 
@@ -495,12 +495,12 @@ __device__ __forceinline__ void roe64(const NodeC<double, D> &L, const NodeC<dou
 // the sides and turning the normal around gives the exact negative.  GEN: the two-point flux is
 // Kennedy-Gruber or Ismail-Roe, else Chandrashekar or Ranocha; `first` orders the sides for the
 // former, which are not written that way.  Lax-Friedrichs dissipation reads the energies u[D + 1] as
-// well (rebuilt from H they would leave a jump of their rounding times the sound speed).  MOM: the
-// nodes hold their momentum, else it is rho v.
-template <int D, int K, bool CV, bool GEN, bool MOM = false>
+// well (rebuilt from H they would leave a jump of their rounding times the sound speed).  mom(left, k): a
+// side's momentum, asked for only where a flux needs it (the central flux, Lax-Friedrichs dissipation).
+template <int D, int K, bool CV, bool GEN, typename Mom>
 __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const NodeC<double, D> &R, double sgn,
                                            const double *n, bool first, const FastConst<double> &fc,
-                                           const PhysConst &pc, double *out)
+                                           const PhysConst &pc, const Mom &mom, double *out)
 {
     const int cf = fc.conv_flux;
     double vnL, vnR;
@@ -536,17 +536,17 @@ __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const Node
         if constexpr (!CV)
             for (int s = 0; s < D + 2; ++s) out[s] *= sgn;
     } else {
-        double mL = L.u[0] * vnL, mR = R.u[0] * vnR;
-        if constexpr (MOM && CV) {
-            mL = L.u[1] * n[0];
-            mR = R.u[1] * n[0];
+        double mL, mR;
+        if constexpr (CV) {
+            mL = mom(true, 0) * n[0];
+            mR = mom(false, 0) * n[0];
             for (int k = 1; k < D; ++k) {
-                mL += L.u[1 + k] * n[k];
-                mR += R.u[1 + k] * n[k];
+                mL += mom(true, k) * n[k];
+                mR += mom(false, k) * n[k];
             }
-        } else if constexpr (MOM) {
-            mL = L.u[1 + K] * sgn;
-            mR = R.u[1 + K] * sgn;
+        } else {
+            mL = mom(true, K) * sgn;
+            mR = mom(false, K) * sgn;
         }
         const double ps = 0.5 * (L.p + R.p);
         out[0] = 0.5 * (mL + mR);
@@ -563,16 +563,22 @@ __device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const Node
         const double hl = 0.5 * fmx<double>(fab<double>(vnL) + L.c, fab<double>(vnR) + R.c);
         out[0] -= hl * (R.u[0] - L.u[0]);
         for (int k = 0; k < D; ++k) {
-            double a = L.u[0] * L.vel[k], b = R.u[0] * R.vel[k];
-            if (MOM) {
-                a = L.u[1 + k];
-                b = R.u[1 + k];
-            }
+            const double a = mom(true, k), b = mom(false, k);
             out[1 + k] -= hl * (b - a);
         }
         out[D + 1] -= hl * (R.u[D + 1] - L.u[D + 1]);
     }
     if (cf == 1 || cf == 5) roe64<D, K, CV>(L, R, sgn, n, vnL, vnR, fc, out);
+}
+
+// The same with the momentum rho v.
+template <int D, int K, bool CV, bool GEN>
+__device__ __forceinline__ void num_flux64(const NodeC<double, D> &L, const NodeC<double, D> &R, double sgn,
+                                           const double *n, bool first, const FastConst<double> &fc,
+                                           const PhysConst &pc, double *out)
+{
+    const auto mom = [&](bool left, int k) { return left ? L.u[0] * L.vel[k] : R.u[0] * R.vel[k]; };
+    num_flux64<D, K, CV, GEN>(L, R, sgn, n, first, fc, pc, mom, out);
 }
 
 // Numerical flux of a face node along the normal sgn * e_K, L the interior

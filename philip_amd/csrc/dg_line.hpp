@@ -1,7 +1,8 @@
 // Line-structured fused stage kernel for the split (two-point) form of the
-// Euler equations on collocated GLL nodes, and of the Navier-Stokes equations
-// on the mixed path (V: the viscous volume and surface terms added to the same
-// items, navier_stokes.cpp / viscous_numerical_flux.cpp).
+// Euler equations on collocated GLL nodes and of the Navier-Stokes equations
+// (V: the viscous volume and surface terms added to the same items,
+// navier_stokes.cpp / viscous_numerical_flux.cpp); in FP64 also for the
+// conservative form (FORM) and on curvilinear grids (CV).
 //
 // The skew-symmetric Hadamard volume term (strong_dg.cpp:1017-1579, Chan 2019
 // eq. 15) couples node a only with the nodes b on its own grid line in each
@@ -20,10 +21,10 @@
 //                     neighbours' face-node states (one item per face node)
 //                     are loaded into LDS, so the line phase makes no global
 //                     loads
-//   L  item-parallel  pair-line items (a line's pairs, sums kept in registers;
-//                     a long line's pairs shared by LS items) and face-node
-//                     items (the surface term, written at once over the face
-//                     node's trace slot); after a barrier the line sums go to
+//   L  item-parallel  face-node items (the surface term, written at once over
+//                     the face node's trace slot) and pair-line items (a line's
+//                     pairs, sums kept in registers; a long line's pairs shared
+//                     by LS items), in which order: FACES_FIRST; after a barrier the line sums go to
 //                     LDS over the (now dead) node cache, one direction at a
 //                     time
 //   E  node-parallel  line partials plus surface terms, FP64 epilogue
@@ -43,8 +44,9 @@ namespace dgx {
 // kernel (held in registers through the line phase) instead of in the epilogue:
 // on for the mixed path (its register budget keeps 4 waves/SIMD), off for FP64,
 // which issues them once the line phase is over instead, so that they are in
-// flight while the line sums go to LDS (TGV p=3 32^3: 220 -> 208 us per stage;
-// p=2 -3 %, p=6 -6 %, p=4 unchanged; at 3D p=5 slower, 366 -> 399 us, so not there).
+// flight while the line sums go to LDS (with the phase order and fluxes before the
+// present ones: 3D p=3 -5 %, p=2 -3 %, p=6 -6 %, p=4 unchanged; p=5 9 % slower, so
+// not there).
 constexpr bool LINE_PREFETCH_RK_F = true;
 constexpr bool LINE_PREFETCH_RK_D = false;
 template <int D, int N> constexpr bool line_late_prefetch_d() { return !(D == 3 && N == 6); }
@@ -60,8 +62,8 @@ template <int D, int N, typename T, int ES = 1, bool V = false, int XJ = LINE_NO
     static constexpr int NP = G::NP, NS = D + 2, NL = G::NL;
     static constexpr int EPB = ES >= 64 ? ES - 64 : ES > 0 ? G::EPB * ES : (G::EPB / -ES > 0 ? G::EPB / -ES : 1);
     static constexpr bool FAST = std::is_same<T, float>::value;
-    // node cache fields: rho, E, vel[D], p, b, |v|^2, sqrt(rho), c, h; FP64: without E (rho h - p)
-    // and |v|^2
+    // node cache fields: rho, E, vel[D], p, b, |v|^2, sqrt(rho), c, h; FP64: rho, vel[D], p, b, h, c,
+    // sqrt(rho), with what node_to_cache64 puts in the place of some
     static constexpr int NQ = FAST ? D + 8 : D + 6;
     // element strides padded to 1 mod 32 words so the stride-N lines of
     // neighbouring elements fall in different LDS banks; FP64 p=1 in 3D, where that padding is a fifth
@@ -136,7 +138,8 @@ template <int D, int N, typename T, bool V> constexpr int line_es()
 template <int D, int N, typename T, bool V> using LineGeoK = LineGeo<D, N, T, line_es<D, N, T, V>(), V>;
 // Waves per SIMD line64_kernel is held to: on curvilinear grids up to p=5 three (stage, held to two ->
 // three: p=4 24^3 207 -> 187 us, p=5 16^3 146 -> 132 us, Navier-Stokes p=5 16^3 272 -> 254 us, p=3 the
-// same); on the box it takes 164 VGPRs at p=5 by itself, and p=6 is slower with a bound.
+// same); held to three the Chandrashekar / Ranocha kernels spill 82 VGPRs at p=4, 62 at p=5 and 66 with
+// the viscous terms.  On the box p=5 takes 159 by itself, and p=6 is slower with a bound.
 template <int D, int N, bool V, bool CV> constexpr int line64_waves() { return CV && N <= 6 ? 3 : 2; }
 
 // ---- node cache in LDS ----------------------------------------------------
@@ -155,10 +158,11 @@ template <int D, int N> __device__ __forceinline__ int qpos(int i)
     }
 }
 
-// A node's cache holds rho, E, the velocity, p, beta, |v|^2, sqrt(rho), c and H (D + 8 values);
-// the momentum is not stored but rebuilt as rho v on load.  Every flux reads nodes in this
-// canonical form (node_canon), whether they come from the cache or from a neighbour trace whose
-// cache is built at the face, so a face evaluates to the same bits in every block layout.
+// A node's cache holds rho, E, the velocity, p, beta, |v|^2, sqrt(rho), c and H (D + 8 values; FP64
+// D + 6, see LineGeo::NQ); the momentum is not stored but rebuilt as rho v on load.  Every mixed flux
+// reads nodes in this canonical form (node_canon), whether they come from the cache or from a
+// neighbour trace whose cache is built at the face, so a face evaluates to the same bits in every
+// block layout; FP64 fluxes read the momentum only where the form or face64 has the state's own.
 
 template <typename T, int D>
 __device__ __forceinline__ void nodef_store(T *q, int st, const NodeC<T, D> &n)
@@ -336,8 +340,6 @@ __device__ __forceinline__ void pairs_f(const Ops1D &ops, const PhysConst &pc, c
     }
 }
 
-// ---- Navier-Stokes terms (either precision) --------------------------------
-
 // FP64, conservative form: node a gets -sum_b D[a][b] F_K(u_b) (CV: contracted with the node's
 // cofactor column), part H of LS of the columns b.
 template <int D, int N, int K, int LS, int H, bool CV>
@@ -361,6 +363,8 @@ __device__ __forceinline__ void cons_line64(const Ops1D &ops, const double *sq, 
         }
     }
 }
+
+// ---- Navier-Stokes terms (either precision) --------------------------------
 
 // Viscous part of the volume term along one line: node a gets -sum_b D[a][b] F_v,K(u_b, q_b)
 // (the conservative D-divergence of strong_dg.cpp:1386-1433 for the dissipative flux); sfv
@@ -531,21 +535,28 @@ __device__ __forceinline__ void face64(const StageArgs &a, const Ops1D &ops, con
         for (int s = 0; s < NS; ++s) qn.u[s] = in.tr[s * in.tst];
         node_fill<double, D>(qn, fc);
     }
-    // the jump of the energy itself (Lax-Friedrichs, SIPG), and of the momentum itself (SIPG, and with
-    // the viscous terms or on a curvilinear grid all but the two-point fluxes without Lax-Friedrichs
-    // dissipation): rebuilt from the cache, they would leave a jump of their own rounding
-    constexpr bool MOM = FORM == FORM_CONS || V || CV;
+    // the jump of the energy itself (Lax-Friedrichs, SIPG) and of the momentum itself (SIPG): rebuilt from
+    // the cache, they would leave a jump of their own rounding
     if (energy_in_sr(pc.conv_flux)) {
         qi.u[D + 1] = qi.sr;
         if (nbl >= 0) qn.u[D + 1] = qn.sr;
     }
-    if ((V && pc.diss_flux == 0) || (MOM && FORM != FORM_CONS && pc.conv_flux != 3 && pc.conv_flux != 5)) {
+    if (V && pc.diss_flux == 0) {
         for (int s = 1; s < NS; ++s) qi.u[s] = a.u[((long)e * NS + s) * NP + fi];
         if (nbl >= 0)
             for (int s = 1; s < NS; ++s) qn.u[s] = a.u[((long)nb * NS + s) * NP + fj];
     }
+    // With the viscous terms or on a curvilinear grid the numerical flux has the states' own momenta too,
+    // read where a flux uses them (read ahead of it: Navier-Stokes p=5 16^3 stage 126-129 -> 130 us).
+    const auto mom = [&](bool left, int k) {
+        if constexpr (FORM == FORM_CONS) return left ? qi.u[1 + k] : qn.u[1 + k];
+        else if constexpr (V || CV)
+            return left ? a.u[((long)e * NS + 1 + k) * NP + fi]
+                        : (nbl >= 0 ? a.u[((long)nb * NS + 1 + k) * NP + fj] : qn.u[1 + k]);
+        else return left ? qi.u[0] * qi.vel[k] : qn.u[0] * qn.vel[k];
+    };
     double fs[NS];
-    num_flux64<D, K, CV, FORM == FORM_GEN, MOM>(qi, qn, sgn, nh, own, fc, pc, fs);
+    num_flux64<D, K, CV, FORM == FORM_GEN>(qi, qn, sgn, nh, own, fc, pc, mom, fs);
     const double iwb = ops.inv_wb;
     const double w = CV ? iwb * area : iwb;
     for (int s = 0; s < NS; ++s) {
@@ -1004,9 +1015,8 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
                          ((!EARLY && a.mode == MODE_LSRK && !a.lsrk_first) ||
                           (butcher_prefetch(D, N, !FAST) && a.mode == MODE_BUTCHER));
     // FP64 at N >= 4: the stage state is read again here for the epilogue (an L2 hit: the block
-    // read it in phase A) instead of being held in registers through the line phase (TGV 32^3
-    // p=3: 177 -> 170 us per stage, 64 -> 16 B/lane of spills; p=4 24^3 294 -> 244 us; at p=2
-    // slower)
+    // read it in phase A) instead of being held in registers through the line phase (measured with
+    // the earlier fluxes: 3D p=3 32^3 -4 %, p=4 24^3 -17 %; at p=2 slower)
     constexpr bool REREAD = !EARLY && LATE_PF && N >= 4;
     double ue[NS];
     if (REREAD && active && a.mode == MODE_LSRK)
@@ -1111,8 +1121,9 @@ line_kernel(StageArgs a, Ops1D ops, PhysConst pc)
 }
 // Waves per SIMD the single-solve 3D line kernel is held to (amdgpu_waves_per_eu; 0: the
 // compiler's choice).  The mixed path at p=3: 4, which it misses by one register otherwise (129).
-// FP64 path: 4 at p=3 (121 VGPRs, TGV 32^3 112 us per stage), 3 at p=4 and p=5 (156 VGPRs, 24^3 144 us
-// and 20^3 183 us; with 4 spills, 226 and 223 us); at p=2 a bound changes nothing and at p=6 it is
+// FP64 path: 4 at p=3 (121 VGPRs, TGV 32^3 112 us per stage), 3 at p=4 and p=5 (168 VGPRs and, with the
+// Chandrashekar / Ranocha fluxes, 116 and 72 spilled; 24^3 144 us and 20^3 183 us, with 4 226 and 223
+// us); at p=2 a bound changes nothing and at p=6 it is
 // slower (16^3, 3: 264 us, the compiler's two waves 247 us), so those keep the compiler's choice.
 template <int D, int N, typename T> constexpr int line_waves()
 {
