@@ -154,7 +154,8 @@ __device__ __forceinline__ void st_cached(double *p, double v)
 // update, Butcher-tableau stage update, or the FSAL error-register accumulation).
 // jac > 0: the node's det J on a curvilinear grid (acc then holds the cofactor-weighted terms):
 // du/dt = acc / J and the un-lifted residual W J du/dt.
-template <int D, int N, typename T>
+// LINE: called by a line kernel.
+template <int D, int N, typename T, bool LINE = false>
 __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &ops, int e, int i, const int *c,
                                                const double *ud, const T *acc, bool use_pf = false,
                                                const double *pf2 = nullptr, const double *pf3 = nullptr,
@@ -196,7 +197,10 @@ __device__ __forceinline__ void stage_epilogue(const StageArgs &a, const Ops1D &
         }
         // the next stage's state, stored to stay in the caches for that stage's read or streamed
         // (store_stays_cached; S2 cached as well: no further gain)
-        if (a.s1_cached)
+        // The mixed 3D line kernels hold the cached store alone: beside the other one it takes 2 us more of
+        // the p=3 32^3 stage's 97.5, wherever the branch stands, against what streaming wins them in a band
+        // around 8.6 MB (p=3 82 -> 78 us a step).
+        if ((LINE && D == 3 && std::is_same<T, float>::value) || a.s1_cached)
             for (int s = 0; s < NS; ++s) st_cached(a.s1_out + base + s * NP, n1[s]);
         else
             for (int s = 0; s < NS; ++s) st_stream(a.s1_out + base + s * NP, n1[s]);

@@ -1084,8 +1084,8 @@ __device__ __forceinline__ void line_block(const StageArgs &a, const Ops1D &ops,
         const T *w = fb + f * NL + node_line<D, N>(k, i);
         for (int s = 0; s < NS; ++s) acc[s] += w[s * LG::NFN];
     }
-    if constexpr (REREAD) stage_epilogue<D, N, T>(a, ops, e, i, c, ue, acc, late_pf, pf2, pf3, jac);
-    else stage_epilogue<D, N, T>(a, ops, e, i, c, ud, acc, pf || late_pf, pf2, pf3, jac);
+    if constexpr (REREAD) stage_epilogue<D, N, T, true>(a, ops, e, i, c, ue, acc, late_pf, pf2, pf3, jac);
+    else stage_epilogue<D, N, T, true>(a, ops, e, i, c, ud, acc, pf || late_pf, pf2, pf3, jac);
 }
 
 // Elements-per-block variant (ES of LineGeo) of the single-solve Euler line kernel: the mixed path
